@@ -129,9 +129,11 @@ static sp_status alloc_levels(sp_ctx* c, Level<T>* lv, bool level0_owned) {
     if ((c->prm.flags & SP_FLAG_CHEBYSHEV) && (s = dmalloc(c, &L.cd, L.n))) return s;
     if (l == 0 && !level0_owned) continue;
     if ((s = dmalloc(c, &L.cx, L.n)) || (s = dmalloc(c, &L.cy, L.n)) || (s = dmalloc(c, &L.cz, L.n)) ||
-        (s = dmalloc(c, &L.e_store, L.n)) || (s = dmalloc(c, &L.b, L.n)) || (s = dmalloc(c, &L.x, L.n)))
+        (s = dmalloc(c, &L.e_store, L.n)))
       return s;
     L.e = L.e_store;
+    // the finest level works on the residual and on a buffer of the z ring
+    if (l > 0 && ((s = dmalloc(c, &L.b, L.n)) || (s = dmalloc(c, &L.x, L.n)))) return s;
   }
   return SP_OK;
 }
@@ -160,19 +162,21 @@ static sp_status ensure_buffers(sp_ctx* c) {
     return s;
   const bool mixed_mg = prec == SP_PREC_MIXED && pc == SP_PRECOND_MG;
   if (mixed_mg) {
-    if ((s = dmalloc(c, &c->r32, N)) || (s = dmalloc(c, &c->z32, N))) return s;
+    float* z;
+    if ((s = dmalloc(c, &c->r32, N)) || (s = dmalloc(c, &z, N))) return s;
+    c->zring[0] = z;
     if ((s = alloc_levels<float>(c, c->lf, true))) return s;
-    // level 0 works on r32 -> z32
     c->lf[0].b = c->r32;
-    c->lf[0].x = c->z32;
+    c->lf[0].x = z;
   } else {
-    if ((s = dmalloc(c, &c->z64, N))) return s;
+    double* z;
+    if ((s = dmalloc(c, &z, N))) return s;
+    c->zring[0] = z;
     c->r32 = nullptr;
-    c->z32 = nullptr;
     if ((s = alloc_levels<double>(c, c->ld, false))) return s;
     Level<double>& L0 = c->ld[0];
     L0.cx = c->cx; L0.cy = c->cy; L0.cz = c->cz; L0.e_store = c->ee; L0.e = c->ee;
-    L0.b = c->r; L0.x = c->z64;
+    L0.b = c->r; L0.x = z;
   }
   // tail: the levels from which every coarser level fits the tail kernel's
   // LDS (seven arrays per level), each finer than the coarsest holding at
@@ -208,6 +212,25 @@ static sp_status ensure_buffers(sp_ctx* c) {
   if ((s = dmalloc(c, &c->wall_var,
                    8 * ((int64_t)D.J * D.K + (int64_t)D.I * D.K + (int64_t)D.I * D.J))))
     return s;
+  // The z ring: as deep as 8 GiB allow (16 buffers up to 512x512x512 in FP32),
+  // and shallower when the device has no room: a solve then forms x more
+  // often.  One allocation for all of it but the first buffer.
+  {
+    const int64_t bytes = N * (mixed_mg ? 4 : 8);
+    const size_t step = ((size_t)bytes + 255) / 256 * 256 + kStagger;
+    c->zdepth = 1;
+    for (int more = (int)std::min<int64_t>(kZRing, ((int64_t)8 << 30) / bytes) - 1; more > 0;
+         more /= 2) {
+      char* z;
+      if (dmalloc(c, &z, step * (size_t)more) != SP_OK) {
+        (void)hipGetLastError();
+        c->last_error.clear();
+        continue;
+      }
+      for (int j = 0; j < more; ++j) c->zring[c->zdepth++] = z + step * (size_t)j;
+      break;
+    }
+  }
   c->allocated_for = (size_t)N;
   c->allocated_prec = prec;
   c->allocated_precond = pc;

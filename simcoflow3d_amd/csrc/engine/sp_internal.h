@@ -15,13 +15,14 @@ constexpr int kMaxLevels = 24;
 constexpr int64_t kTailCells = 512;  // levels this small run in one workgroup
 constexpr int kTailLdsBytes = 144 * 1024;  // LDS of that workgroup (7 arrays per level)
 constexpr int kRedBlockThreads = 256;
+constexpr int kZRing = 16;  // preconditioned residuals kept before x is formed from them
 
 // Scalars of the outer CG, resident in device memory so no host round trip
 // is needed between the kernels of one iteration.
 struct Scalars {
   double rz;        // (r, z) of the current iteration
   double alpha, beta;
-  double pq, zq;
+  double pq;
   double rmax;      // max |r_i| / V_i of the recursive residual
   double bmean;     // mean of b over active cells (singular systems)
   double bsum, esum, bmax, shift, divmax;
@@ -31,13 +32,15 @@ struct Scalars {
   double src_max;   // max |pbar_i| / V_i of the adjoint source
   double rsum, qsum;  // sums of r and q over the cells (for the z shift)
   double npart[8];  // scratch results of small reductions
+  // alpha, beta and the shift of z of the CG steps whose z are kept
+  double hist_alpha[kZRing], hist_beta[kZRing], hist_m[kZRing];
   int64_t active;
   int32_t done;     // 1 once converged (kernels then return immediately)
   int32_t iter;
   int32_t first;
   int32_t nonfinite;
   int32_t singular;
-  int32_t pad;
+  int32_t nhist;    // number of those steps
   uint32_t counter[16];  // last-block counters, one per reduction site
   uint32_t stale_count;  // GFM faces that need the previous-beta fixup
   uint32_t pad2[3];
@@ -114,7 +117,7 @@ struct sp_ctx {
   int device = 0;
   int num_cu = 256;  // compute units of the device (workgroup sizing)
   int desc_state = -1;      // has_e of the uploaded level table, -1: stale
-  bool fuse_dots = false;  // the finest post-smoother also forms (r,z), (z,q), (dw,z)
+  bool fuse_dots = false;  // the finest post-smoother also forms (r,z), (dw,z)
   uint32_t dots_nb = 0;    // workgroups of that post-smoother (its partials)
   hipStream_t stream = nullptr;
   sp::Dims dm{};
@@ -138,12 +141,16 @@ struct sp_ctx {
   bool has_e = false;
 
   // CG vectors (FP64)
-  double *x = nullptr, *r = nullptr, *q = nullptr, *p0 = nullptr, *p1 = nullptr, *z64 = nullptr;
+  double *x = nullptr, *r = nullptr, *q = nullptr, *p0 = nullptr, *p1 = nullptr;
   // iterative refinement of non-singular systems: pressure = x + xd, xe the
   // increment being solved for, p1 its right-hand side
   double *xd = nullptr, *xe = nullptr;
   bool xd_active = false;
-  float *r32 = nullptr, *z32 = nullptr;
+  float* r32 = nullptr;
+  // preconditioned residuals of the last CG steps (FP32 with an FP32 V-cycle),
+  // zdepth of them; zring[0] always exists
+  void* zring[sp::kZRing] = {};
+  int zdepth = 0;
 
   // multigrid hierarchies (only one is populated, by precision)
   int levels = 0;

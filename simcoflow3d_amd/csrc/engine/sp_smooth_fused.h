@@ -45,11 +45,10 @@ struct FusedArgs {
   int cnx, cny;
   int kchunk;    // even
   T omega;       // over-relaxation: x += omega (x_gs - x)
-  // finest post-smoother only: the CG dot products (r,z), (z,q), (dw,z) of
-  // the z it writes, as per-workgroup partials (r and the diagonal weight:
-  // the FP32 right-hand side and diagonal the leg already holds)
+  // finest post-smoother only: the CG dot products (r,z), (dw,z) of the z it
+  // writes, as per-workgroup partials (r and the diagonal weight: the FP32
+  // right-hand side and diagonal the leg already holds)
   int dots;
-  const double* dq;
   RedSite dsite;
 };
 
@@ -102,7 +101,6 @@ template <typename T>
 struct PlaneLoad {
   T b, cx, cy, cz, cxm, cym, e, xin, xc;
   bool vt;
-  double dq;  // dot-product input of the step's output plane t - H
 };
 
 // Per-thread constants of the march.
@@ -117,7 +115,7 @@ struct FusedCol {
   uint32_t cplane;       // post: bytes per coarse plane
 };
 
-template <typename T, int MODE, bool HAS_E, bool DOTS, int H>
+template <typename T, int MODE, bool HAS_E>
 __device__ inline void load_plane(PlaneLoad<T>& L, const FusedArgs<T>& A, const FusedCol& C, int t) {
   const int tc = t < 0 ? 0 : (t >= A.nz ? A.nz - 1 : t);
   const uint32_t n = C.col + C.plane * (uint32_t)tc;
@@ -136,13 +134,6 @@ __device__ inline void load_plane(PlaneLoad<T>& L, const FusedArgs<T>& A, const 
     L.xin = T(0);
     L.xc = T(0);
   }
-  // with the plane loads, so the in-order load counter never makes a step
-  // wait for planes fetched after them
-  if (DOTS && A.dots && C.tile && C.in_ij) {
-    const int q = t - H, qc = q < 0 ? 0 : (q >= A.nz ? A.nz - 1 : q);
-    const uint32_t e = C.col / (uint32_t)sizeof(T) + (C.plane / (uint32_t)sizeof(T)) * (uint32_t)qc;
-    L.dq = at_off(A.dq, e * 8u);
-  }
 }
 
 // Register windows along k.  Logical plane o (0 = newest) of step u lives in
@@ -154,7 +145,7 @@ struct FusedState {
   T xw[W], bw[W], dw[W], rdw[W], czw[W], cxw[W], cxmw[W], cyw[W], cymw[W];
   bool dpos[W];  // d > 0 of each plane, tested once when the plane enters
   T racc;
-  double dacc[3];  // CG dot products (finest post-smoother)
+  double dacc[2];  // CG dot products (finest post-smoother)
 };
 
 // One pipeline step: plane t enters (from L), half-sweeps on the planes
@@ -256,8 +247,7 @@ __device__ inline void fused_step(FusedState<T, NU, MODE>& F, const PlaneLoad<T>
       // rz rounded at 1e-7 only perturbs the step length, and the x and r
       // updates stay consistent (both use the same alpha)
       F.dacc[0] += (double)F.bw[S(H)] * z;
-      F.dacc[1] += z * L.dq;
-      F.dacc[2] += (double)F.dw[S(H)] * z;
+      F.dacc[1] += (double)F.dw[S(H)] * z;
     }
   }
   lds_barrier();
@@ -302,7 +292,7 @@ __device__ inline void march_steps(FusedState<T, NU, MODE>& F, PlaneLoad<T> (&LB
     static_assert(FusedShape<NU>::W % P == 0, "load buffers must tile the window");
     PlaneLoad<T>& L = LB[U % P];
     fused_step<T, NU, MODE, HAS_E, DOTS, U, EX, EY>(F, L, A, C, xs, rs, t + U, k0, k1);
-    load_plane<T, MODE, HAS_E, DOTS, FusedShape<NU>::H>(L, A, C, t + U + P);
+    load_plane<T, MODE, HAS_E>(L, A, C, t + U + P);
     march_steps<T, NU, MODE, HAS_E, DOTS, CHECK, U + 1, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   }
 }
@@ -343,7 +333,7 @@ __global__ void __launch_bounds__(EX * EY) k_smooth_fused(FusedArgs<T> A, const 
     F.dpos[o] = false;
   }
   F.racc = T(0);
-  F.dacc[0] = F.dacc[1] = F.dacc[2] = 0.0;
+  F.dacc[0] = F.dacc[1] = 0.0;
   for (int q = C.ty * EX + C.tx; q < R * (EY + 2) * (EX + 2); q += EX * EY) (&xs[0][0][0])[q] = T(0);
   for (int q = C.ty * EX + C.tx; q < 2 * EY * EX; q += EX * EY) (&rs[0][0][0])[q] = T(0);
   // cz of the plane below the first loaded one (bottom face of that plane):
@@ -360,14 +350,14 @@ __global__ void __launch_bounds__(EX * EY) k_smooth_fused(FusedArgs<T> A, const 
   constexpr bool DOTS = FINE && MODE == 1 && sizeof(T) == 4;  // FP64: separate dots kernel
   PlaneLoad<T> LB[P];
 #pragma unroll
-  for (int u = 0; u < P; ++u) load_plane<T, MODE, HAS_E, DOTS, H>(LB[u], A, C, t0 + u);
+  for (int u = 0; u < P; ++u) load_plane<T, MODE, HAS_E>(LB[u], A, C, t0 + u);
   int t = t0;
   for (; t + W <= t1; t += W)
     march_steps<T, NU, MODE, HAS_E, DOTS, false, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   if (t < t1)
     march_steps<T, NU, MODE, HAS_E, DOTS, true, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   if constexpr (DOTS) {
-    if (A.dots) block_partials<EX * EY, 3, 0u>(A.dsite, F.dacc);
+    if (A.dots) block_partials<EX * EY, 2, 0u>(A.dsite, F.dacc);
   }
 }
 

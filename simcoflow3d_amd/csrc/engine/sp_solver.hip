@@ -6,6 +6,14 @@
 // host only polls a convergence flag the finalize kernel writes into pinned
 // host memory, one iteration behind.
 //
+// The search direction p and the iterate x are not carried through the
+// iterations.  With p_k = z_k - m_k + beta_k p_{k-1} the CG needs p only in
+// q = A p (a recurrence of its own, q_k = A (z_k - m_k) + beta_k q_{k-1}), in
+// (p, q), which equals (z - m, q) because beta makes the new direction
+// A-orthogonal to the last one, and in x, which is a combination of the z_k.
+// So the preconditioned residuals are kept (kZRing of them) and x is formed
+// from them in one pass at the end.
+//
 // Multigrid: cell-centred coarsening by 2, piecewise-constant transfers
 // (restriction = sum over children, prolongation = injection), coarse face
 // coefficients = scale * sum of the fine face coefficients they cover (the
@@ -186,6 +194,7 @@ struct TailArgs {
   int pre, post, coarse_sweeps, singular, has_e;
   T omega, omega_c;  // over-relaxation of the Gauss-Seidel updates (level 0, coarser)
   const LevelView<T>* lv;   // the levels in global memory
+  T* x;                     // x of the first tail level
   int off[kMaxLevels];      // element offset of each tail level in LDS
 };
 
@@ -438,7 +447,7 @@ __global__ void __launch_bounds__(1024) k_tail(TailArgs<T> A, const Scalars* S) 
     const LevelView<T> G = A.lv[A.first];
     const TailLevel<T> V = tail_level(lds, A, A.first);
     const int n = G.nx * G.ny * G.nz;
-    for (int q = threadIdx.x; q < n; q += blockDim.x) G.x[q] = V.x[q];
+    for (int q = threadIdx.x; q < n; q += blockDim.x) A.x[q] = V.x[q];
   }
 }
 
@@ -476,7 +485,8 @@ struct CgArgs {
   const double *dxp, *dyp, *dzp;
   const double* b;
   double *x, *r, *q;
-  double* p;  // search direction
+  double* p;  // search direction at the last pass that formed x
+  int slot;   // this iteration's entry in the history of z, beta, m and alpha
   double* z64;  // written by the Jacobi preconditioner only
   const float* z32;
   float* r32;
@@ -566,8 +576,8 @@ __global__ void __launch_bounds__(256) k_cg_jacobi(CgArgs A) {
   }
 }
 
-// r = b - mean(b) - A x  (x = 0 when from_zero); resets p and q.  KC cells
-// of a column per thread, the mask and b of all of them loaded first (cell
+// r = b - mean(b) - A x  (x = 0, not read, when from_zero).  KC cells of a
+// column per thread, the mask and b of all of them loaded first (cell
 // index clamped into the column).
 template <int KC>
 __global__ void __launch_bounds__(256) k_cg_residual(CgArgs A, int from_zero) {
@@ -605,9 +615,6 @@ __global__ void __launch_bounds__(256) k_cg_residual(CgArgs A, int from_zero) {
       }
       A.r[n] = rv;
       if (A.r32) A.r32[n] = (float)rv;
-      if (from_zero) A.x[n] = 0.0;
-      A.q[n] = 0.0;
-      A.p[n] = 0.0;
     }
   }
   block_partials<kTileThreads, 3, 3u>(A.site, v);
@@ -622,7 +629,8 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_residual_fin(CgArgs A, uint3
     Scalars* S = A.S;
     S->rmax = out[0];
     S->rsum = out[2];
-    S->qsum = 0.0;  // q was reset
+    S->qsum = 0.0;
+    S->nhist = 0;
     S->nonfinite = S->nonfinite || out[1] > 0.0 || !is_finite(out[0]);
     S->done = (out[0] <= A.tol || S->nonfinite) ? 1 : 0;
     S->first = 1;
@@ -633,6 +641,17 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_residual_fin(CgArgs A, uint3
   }
 }
 
+// The scalars of the new search direction p = (z - m) + beta p_old.
+__device__ inline void set_direction(Scalars* S, int slot, double m, double rz, double beta) {
+  S->zshift = m;
+  S->beta = beta;
+  S->rz = rz;
+  S->first = 0;
+  S->hist_m[slot] = m;
+  S->hist_beta[slot] = beta;
+  if (!is_finite(rz) || !is_finite(beta)) { S->nonfinite = 1; S->done = 1; }
+}
+
 // rz = (r, z), zq = (z, q);  beta = -alpha zq / rz_old (flexible CG).
 // Singular systems: z is shifted by its diagonal-weighted mean m so the
 // iterate keeps the pressure of the stiff (high-coefficient) phase near zero;
@@ -641,6 +660,7 @@ __global__ void __launch_bounds__(256) k_cg_dots(CgArgs A) {
   Scalars* S = A.S;
   if (S->done) return;
   const Col3 q = col_of(A.I, A.J, A.K);
+  const bool first = S->first != 0;  // q is not written before the first product
   double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (q.in) {
     const int64_t IJ = (int64_t)A.I * A.J;
@@ -648,7 +668,7 @@ __global__ void __launch_bounds__(256) k_cg_dots(CgArgs A) {
 #pragma unroll 4
     for (int c = q.c0; c < q.c1; ++c, n += IJ) {
       if (A.active[n]) {
-        const double z = zval(A, n), r = A.r[n], qq = A.q[n];
+        const double z = zval(A, n), r = A.r[n], qq = first ? 0.0 : A.q[n];
         v[0] += r * z;
         v[1] += z * qq;
         v[2] += (double)A.dw[n] * z;
@@ -668,51 +688,42 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_dots_fin(CgArgs A, uint32_t 
   if (flat_tid() == 0) {
     const double m = (S->singular && S->dsum > 0.0) ? t[2] / S->dsum : 0.0;
     const double rzm = t[0] - m * t[3], zqm = t[1] - m * t[4];
-    S->zshift = m;
-    S->beta = S->first ? 0.0 : -S->alpha * zqm / S->rz;
-    S->rz = rzm;
-    S->zq = zqm;
-    S->first = 0;
-    if (!is_finite(rzm) || !is_finite(S->beta)) { S->nonfinite = 1; S->done = 1; }
+    set_direction(S, A.slot, m, rzm, S->first ? 0.0 : -S->alpha * zqm / S->rz);
   }
 }
 
-// Same as k_cg_dots_fin with (r,z), (z,q), (dw,z) from the finest
-// post-smoother's partials and the sums of r and q from the update and the
-// SpMV of the previous iteration.
-__global__ void __launch_bounds__(kFinThreads) k_cg_dots3_fin(CgArgs A, uint32_t nb) {
+// Same as k_cg_dots_fin behind the fused V-cycle: (r,z) and (dw,z) from the
+// finest post-smoother's partials, the sum of r from the update.  That V-cycle
+// is a fixed symmetric operator up to its own rounding (pre: red, black,
+// post: black, red, restriction the transpose of the prolongation), so z is
+// orthogonal to the previous residual and beta = rz / rz_old needs no (z,q):
+// the leg does not have to read q.
+__global__ void __launch_bounds__(kFinThreads) k_cg_dots2_fin(CgArgs A, uint32_t nb) {
   Scalars* S = A.S;
   if (S->done) return;
-  double t[3];
-  finalize_partials<kFinThreads, 3, 0u>(A.site, nb, t);
+  double t[2];
+  finalize_partials<kFinThreads, 2, 0u>(A.site, nb, t);
   if (flat_tid() == 0) {
-    const double m = (S->singular && S->dsum > 0.0) ? t[2] / S->dsum : 0.0;
-    const double rzm = t[0] - m * S->rsum, zqm = t[1] - m * S->qsum;
-    S->zshift = m;
-    S->beta = S->first ? 0.0 : -S->alpha * zqm / S->rz;
-    S->rz = rzm;
-    S->zq = zqm;
-    S->first = 0;
-    if (!is_finite(rzm) || !is_finite(S->beta)) { S->nonfinite = 1; S->done = 1; }
+    const double m = (S->singular && S->dsum > 0.0) ? t[1] / S->dsum : 0.0;
+    const double rzm = t[0] - m * S->rsum;
+    set_direction(S, A.slot, m, rzm, S->first ? 0.0 : rzm / S->rz);
   }
 }
 
-// The search direction and its image in one pass:
-//   x += alpha p_old            (the x half of the previous CG step)
-//   p = (z - m) + beta p_old,   q = A p = A z - m e + beta q_old
-// on active cells (0 elsewhere), with (p, q) and sum q for alpha.  A 1 is the
-// diagonal-only term e on active rows (the face couplings of a row sum to its
-// diagonal minus e), so the stencil is applied to z, which is complete in
-// memory, and p and q need no neighbours.  Each thread walks its column
-// keeping z and the z-coupling of planes k-1 / k / k+1 in registers.  After
-// the last CG step k_cg_xflush applies its x half.
+// The image of the search direction in one pass:
+//   q = A (z - m) + beta q_old
+// with (p, q) = (z - m, q) and sum q for alpha.  A 1 is the diagonal-only
+// term e (the face couplings of a row sum to its diagonal minus e), so the
+// stencil is applied to z, which is complete in memory.  Rows of inactive
+// cells have no couplings and z = 0: q stays 0 there without a mask.  Each
+// thread walks its column keeping z and the z-coupling of planes k-1 / k /
+// k+1 in registers.
 template <typename Z>
-__global__ void __launch_bounds__(256) k_cg_pspmv(CgArgs A, const Z* zv) {
+__global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
   Scalars* S = A.S;
   if (S->done) return;
   const Col3 q = col_of(A.I, A.J, A.K);
-  const double alpha = S->alpha;
-  double v[2] = {0.0, 0.0};  // (p, q), sum q
+  double v[2] = {0.0, 0.0};  // (z - m, q), sum q
   if (q.in) {
     const double beta = S->beta, m = S->zshift;
     const int64_t I = A.I, IJ = (int64_t)A.I * A.J;
@@ -734,6 +745,7 @@ __global__ void __launch_bounds__(256) k_cg_pspmv(CgArgs A, const Z* zv) {
       const double zw = (double)zv[n - dW], ze = (double)zv[n + dE];
       const double zs = (double)zv[n - dS], zn = (double)zv[n + dN];
       const double en = A.e ? A.e[n] : 0.0;
+      const double qo = beta != 0.0 ? A.q[n] : 0.0;  // not written before the first product
       double d = cxm + cym;
       d = d + czm;
       d = d + cx;
@@ -747,14 +759,9 @@ __global__ void __launch_bounds__(256) k_cg_pspmv(CgArgs A, const Z* zv) {
       az -= cx * ze;
       az -= cy * zn;
       az -= cz * zp;
-      const bool act = A.active[n] != 0;
-      const double po = A.p[n];
-      A.x[n] += alpha * po;
-      const double pv = act ? (zc - m) + beta * po : 0.0;
-      const double qv = act ? (az - m * en) + beta * A.q[n] : 0.0;
-      A.p[n] = pv;
+      const double qv = (az - m * en) + beta * qo;
       A.q[n] = qv;
-      v[0] += pv * qv;
+      v[0] += (zc - m) * qv;
       v[1] += qv;
       zm = zc;
       zc = zp;
@@ -773,12 +780,13 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_spmv_fin(CgArgs A, uint32_t 
     S->pq = t[0];
     S->qsum = t[1];
     S->alpha = S->rz / t[0];
+    S->hist_alpha[A.slot] = S->alpha;
+    S->nhist = A.slot + 1;
     if (!is_finite(S->alpha)) { S->nonfinite = 1; S->done = 1; }
   }
 }
 
-// r -= alpha q ; rmax = max |r|/V (x += alpha p follows in the next
-// k_cg_pspmv, or in k_cg_xflush after the last step)
+// r -= alpha q ; rmax = max |r|/V
 __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
   Scalars* S = A.S;
   if (S->done) return;
@@ -802,19 +810,80 @@ __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
   block_partials<kTileThreads, 2, 1u>(A.site, v);
 }
 
-// x += alpha p of the last CG step (its r update is done; the k_cg_pspmv
-// that would apply it is never launched, or returns once the loop is done).
-// alpha = 0 and p = 0 after a residual that already meets the tolerance.
-__global__ void __launch_bounds__(256) k_cg_xflush(CgArgs A) {
+// x from the kept z of the steps since the last such pass:
+//   x_new = x + sum_j gamma_j (z_j - m_j) + gamma_b p,
+//   gamma_last = alpha_last,  gamma_j = alpha_j + beta_{j+1} gamma_{j+1},
+//   gamma_b = beta_0 gamma_0,
+// on active cells (0 elsewhere), from x = 0 when `assign`.  m is taken off
+// each z before the sum: in a two-phase system the stiff phase's z sits close
+// to m, and its differences matter.  With `keep_p` (a full history in the
+// middle of a solve) p becomes the current direction, from the same z.
+// z, x and the mask are read and x is written once: 15 steps of an FP32
+// V-cycle at 256^3 move 69 B a cell here, where carrying x and p through the
+// iterations moved 32 B a cell in each of them.
+template <typename Z>
+struct ZHist {
+  const Z* z[kZRing];
+};
+constexpr int kFlushCells = 4;  // cells per thread
+template <typename Z>
+__global__ void __launch_bounds__(256) k_cg_xflush(CgArgs A, ZHist<Z> H, int64_t N, int assign,
+                                                   int keep_p) {
   const Scalars* S = A.S;
-  const Col3 q = col_of(A.I, A.J, A.K);
-  if (!q.in) return;
-  const double alpha = S->alpha;
-  const int64_t IJ = (int64_t)A.I * A.J;
-  int64_t n = q.a + (int64_t)A.I * (q.b + (int64_t)A.J * q.c0);
+  __shared__ double gam[kZRing], pi[kZRing], sm[kZRing], base[2];
+  const int nh = S->nhist;
+  if (threadIdx.x == 0) {
+    double g = 0.0, w = 1.0;
+    for (int j = nh - 1; j >= 0; --j) {
+      g = S->hist_alpha[j] + g;
+      gam[j] = g;
+      pi[j] = w;
+      sm[j] = S->hist_m[j];
+      g *= S->hist_beta[j];
+      w *= S->hist_beta[j];
+    }
+    base[0] = g;
+    base[1] = w;
+  }
+  __syncthreads();
+  const int64_t n0 = (int64_t)blockIdx.x * (256 * kFlushCells) + threadIdx.x;
+  double xa[kFlushCells], pa[kFlushCells];
+  bool act[kFlushCells];
+  const double gb = nh > 0 ? base[0] : 0.0, pb = base[1];
+#pragma unroll
+  for (int u = 0; u < kFlushCells; ++u) {
+    const int64_t n = min(n0 + 256 * u, N - 1);
+    act[u] = A.active[n] != 0;
+    xa[u] = assign ? 0.0 : A.x[n];
+    pa[u] = 0.0;
+    // beta of a solve's first step is 0, and p is not written before
+    if (gb != 0.0 || (keep_p && pb != 0.0)) {
+      const double p = A.p[n];
+      xa[u] += gb * p;
+      pa[u] = pb * p;
+    }
+  }
 #pragma unroll 4
-  for (int c = q.c0; c < q.c1; ++c, n += IJ) A.x[n] += alpha * A.p[n];
+  for (int j = 0; j < nh; ++j) {
+    const double g = gam[j], w = pi[j], m = sm[j];
+    const Z* z = H.z[j];
+#pragma unroll
+    for (int u = 0; u < kFlushCells; ++u) {
+      const int64_t n = min(n0 + 256 * u, N - 1);
+      const double zv = (double)z[n] - m;
+      xa[u] += g * zv;
+      pa[u] += w * zv;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kFlushCells; ++u) {
+    const int64_t n = n0 + 256 * u;
+    if (n >= N) break;
+    A.x[n] = act[u] ? xa[u] : 0.0;
+    if (keep_p) A.p[n] = act[u] ? pa[u] : 0.0;
+  }
 }
+__global__ void k_cg_hist_reset(Scalars* S) { S->nhist = 0; }
 
 __global__ void __launch_bounds__(kFinThreads) k_cg_update_fin(CgArgs A, uint32_t nb) {
   Scalars* S = A.S;
@@ -929,13 +998,11 @@ void launch_fused_tile(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine,
   int slot;
   if (A.dots) c->dots_nb = grd.x * grd.y * grd.z;
   // algorithmic words per cell: pre b + 3 faces -> x (+ coarse b);
-  // post x_pre + 3 faces + b -> x (+ coarse x); the dot products add q
-  // (FP64)
+  // post x_pre + 3 faces + b -> x (+ coarse x)
   const double words = mode == 0 ? 5.0 + 0.125 : 6.0 + 0.125;
   timer_begin(c, fine ? (mode == 0 ? "mg_pre_fine" : "mg_post_fine")
                       : (mode == 0 ? "mg_pre_coarse" : "mg_post_coarse"),
-              level_bytes(L, words + (L.e ? 1.0 : 0.0)) + (A.dots ? 8.0 * (double)L.n : 0.0),
-              &slot);
+              level_bytes(L, words + (L.e ? 1.0 : 0.0)), &slot);
   const Scalars* S = c->S;
 #define SP_FUSED_LAUNCH(MODE_, FINE_)                                                         \
   do {                                                                                        \
@@ -971,7 +1038,6 @@ void launch_fused(sp_ctx* c, Level<T>* lv, int l, int mode) {
   else { A.xin = L.xs; A.xc = C.x; A.xout = L.x; }
   if (mode == 1 && l == 0 && c->fuse_dots) {
     A.dots = 1;
-    A.dq = c->q;
     A.dsite = red_site(c, kSiteDots);
   }
   const bool fine = l == 0;
@@ -1051,6 +1117,7 @@ void vcycle(sp_ctx* c, Level<T>* lv) {
     A.singular = c->S_host->singular;
     A.has_e = lv[Lt].e ? 1 : 0;
     A.lv = reinterpret_cast<const LevelView<T>*>(c->mg_desc);
+    A.x = lv[Lt].x;
     int64_t off = 0;
     for (int l = 0; l < kMaxLevels; ++l) {
       A.off[l] = (int)off;
@@ -1153,10 +1220,7 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
   A.hflag = c->hflags_dev;
   A.tol = tol;
   if (mixed && mg) {
-    A.z32 = c->z32;
     A.r32 = c->r32;
-  } else {
-    A.z64 = c->z64;
   }
   int slot;
   const double NB = (double)D.N;
@@ -1179,14 +1243,22 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
   };
   auto enqueue_residual = [&](int from_zero) {
     A.site = red_site(c, kSiteResidual);
-    timer_begin(c, "cg_residual", NB * (from_zero ? 8 + 1 + 8 * 4 : 8 * 5 + eb + 1 + 8 * 4),
+    timer_begin(c, "cg_residual", NB * ((from_zero ? 8 + 1 : 8 * 5 + eb + 1) + 8 + (A.r32 ? 4 : 0)),
                 &slot);
     hipLaunchKernelGGL(k_cg_residual<kResK>, col_grid_k<kResK>(D.I, D.J, D.K), blk, 0, c->stream,
                        A, from_zero);
     timer_end(c, slot);
     finalize(k_cg_residual_fin, kSiteResidual, col_blocks_k<kResK>(D.I, D.J, D.K));
   };
+  // z of this step goes into its buffer of the ring
   auto precondition = [&]() {
+    if (mixed && mg) {
+      c->lf[0].x = static_cast<float*>(c->zring[A.slot]);
+      A.z32 = c->lf[0].x;
+    } else {
+      A.z64 = static_cast<double*>(c->zring[A.slot]);
+      if (mg) c->ld[0].x = A.z64;
+    }
     if (mg) {
       if (mixed) vcycle<float>(c, c->lf);
       else vcycle<double>(c, c->ld);
@@ -1216,6 +1288,28 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
   } else {
     enqueue_residual(1);
   }
+  // x from the kept z (k_cg_xflush); `keep_p`: the solve goes on
+  bool assign = !resume;
+  auto form_x = [&](bool keep_p) {
+    const dim3 grd((unsigned)((D.N + 256 * kFlushCells - 1) / (256 * kFlushCells)));
+    // counts a full history; the last pass of a solve reads what it holds
+    timer_begin(c, "cg_xflush", NB * (zb * c->zdepth + 1 + (assign ? 8 : 16) + (keep_p ? 8 : 0)),
+                &slot);
+    if (mixed && mg) {
+      ZHist<float> H{};
+      for (int j = 0; j < c->zdepth; ++j) H.z[j] = static_cast<const float*>(c->zring[j]);
+      hipLaunchKernelGGL(k_cg_xflush<float>, grd, dim3(256), 0, c->stream, A, H, D.N,
+                         assign ? 1 : 0, keep_p ? 1 : 0);
+    } else {
+      ZHist<double> H{};
+      for (int j = 0; j < c->zdepth; ++j) H.z[j] = static_cast<const double*>(c->zring[j]);
+      hipLaunchKernelGGL(k_cg_xflush<double>, grd, dim3(256), 0, c->stream, A, H, D.N,
+                         assign ? 1 : 0, keep_p ? 1 : 0);
+    }
+    timer_end(c, slot);
+    if (keep_p) hipLaunchKernelGGL(k_cg_hist_reset, dim3(1), dim3(1), 0, c->stream, c->S);
+    assign = false;
+  };
   int restarts = 0;
   const int max_iter = std::max(1, c->prm.max_iter);
   bool finished = false;
@@ -1224,22 +1318,28 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
     // flag written at the end of iteration `it - 1`
     bool prev_pending = false;
     int cur = 0;
+    A.slot = 0;
     while (it < max_iter) {
+      if (A.slot == c->zdepth) {  // the ring is full and the solve goes on
+        form_x(true);
+        A.slot = 0;
+      }
       precondition();
       if (c->fuse_dots) {
-        finalize(k_cg_dots3_fin, kSiteDots, c->dots_nb);
+        finalize(k_cg_dots2_fin, kSiteDots, c->dots_nb);
       } else {
         launch_col(k_cg_dots, kSiteDots, "cg_dots", NB * (8 + zb + 8 + 4 + 1));
         finalize(k_cg_dots_fin, kSiteDots, ncol);
       }
-      // z (stencil), p, q, three couplings, e, mask -> p, q
+      // z (stencil), q, three couplings, e -> q
       {
         A.site = red_site(c, kSiteSpmv);
-        timer_begin(c, "cg_pspmv", NB * (zb + 8 + 8 + 8 + 24 + eb + 1 + 8 + 8 + 8), &slot);
+        timer_begin(c, "cg_spmv", NB * (zb + 8 + 24 + eb + 8), &slot);
         if (A.z32)
-          hipLaunchKernelGGL(k_cg_pspmv<float>, cgrd, blk, 0, c->stream, A, (const float*)A.z32);
+          hipLaunchKernelGGL(k_cg_spmv<float>, cgrd, blk, 0, c->stream, A, (const float*)A.z32);
         else
-          hipLaunchKernelGGL(k_cg_pspmv<double>, cgrd, blk, 0, c->stream, A, A.z64);
+          hipLaunchKernelGGL(k_cg_spmv<double>, cgrd, blk, 0, c->stream, A,
+                             (const double*)A.z64);
         timer_end(c, slot);
       }
       finalize(k_cg_spmv_fin, kSiteSpmv, ncol);
@@ -1247,6 +1347,7 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
       finalize(k_cg_update_fin, kSiteUpdate, ncol);
       hipEventRecord(evs[cur], c->stream);
       ++it;
+      ++A.slot;
       if (prev_pending) {
         e = hipEventSynchronize(evs[cur ^ 1]);
         if (e != hipSuccess) { hipEventDestroy(evs[0]); hipEventDestroy(evs[1]); return hip_check(c, e, "solve"); }
@@ -1255,8 +1356,7 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
       prev_pending = true;
       cur ^= 1;
     }
-    // x += alpha p of the last step
-    launch_col(k_cg_xflush, kSiteUpdate, "cg_xflush", NB * 24);
+    form_x(false);
     e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) { hipEventDestroy(evs[0]); hipEventDestroy(evs[1]); return hip_check(c, e, "solve"); }
     e = hipMemcpy(c->S_host, c->S, sizeof(Scalars), hipMemcpyDeviceToHost);
