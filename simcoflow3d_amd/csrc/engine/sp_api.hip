@@ -150,7 +150,6 @@ static sp_status ensure_buffers(sp_ctx* c) {
     return SP_OK;
   free_buffers(c);
   c->levels = L;
-  c->desc_state = -1;  // level table must be uploaded again
   const int64_t N = D.N;
   sp_status s;
   if ((s = dmalloc(c, &c->pocoef, 6 * N)) || (s = dmalloc(c, &c->cx, N)) || (s = dmalloc(c, &c->cy, N)) ||
@@ -178,23 +177,7 @@ static sp_status ensure_buffers(sp_ctx* c) {
     L0.cx = c->cx; L0.cy = c->cy; L0.cz = c->cz; L0.e_store = c->ee; L0.e = c->ee;
     L0.b = c->r; L0.x = z;
   }
-  // tail: the levels from which every coarser level fits the tail kernel's
-  // LDS (seven arrays per level), each finer than the coarsest holding at
-  // most kTailCells cells.  c->levels when not even the coarsest level fits
-  // (a hierarchy cut short by mg_levels, or a large grid that cannot
-  // coarsen): the V-cycle then smooths the coarsest level in global memory.
-  {
-    const int64_t esz = mixed_mg ? 4 : 8;
-    c->tail_level = c->levels;
-    int64_t bytes = 0;
-    for (int l = c->levels - 1; l >= 0; --l) {
-      const int64_t n = mixed_mg ? c->lf[l].n : c->ld[l].n;
-      bytes += 7 * esz * n;
-      if (bytes > kTailLdsBytes || (l < c->levels - 1 && n > kTailCells)) break;
-      c->tail_level = l;
-    }
-  }
-  if ((s = dmalloc(c, reinterpret_cast<char**>(&c->mg_desc), 128 * kMaxLevels))) return s;
+  mg_tail_level(c, mixed_mg);
   c->stale_cap = std::min<int64_t>(6 * N, std::max<int64_t>(1 << 20, N / 2));
   if ((s = dmalloc(c, &c->stale_list, 3 * c->stale_cap))) return s;
   if ((s = dmalloc(c, &c->col_last, 12 * (int64_t)D.I * D.J)) ||

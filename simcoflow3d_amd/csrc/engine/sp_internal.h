@@ -12,8 +12,7 @@
 namespace sp {
 
 constexpr int kMaxLevels = 24;
-constexpr int64_t kTailCells = 512;  // levels this small run in one workgroup
-constexpr int kTailLdsBytes = 144 * 1024;  // LDS of that workgroup (7 arrays per level)
+constexpr int kTailLdsBytes = 144 * 1024;  // LDS of the V-cycle's tail workgroup
 constexpr int kRedBlockThreads = 256;
 constexpr int kZRing = 16;  // preconditioned residuals kept before x is formed from them
 
@@ -116,7 +115,6 @@ struct sp_ctx {
   sp_params prm;
   int device = 0;
   int num_cu = 256;  // compute units of the device (workgroup sizing)
-  int desc_state = -1;      // has_e of the uploaded level table, -1: stale
   bool fuse_dots = false;  // the finest post-smoother also forms (r,z), (dw,z)
   uint32_t dots_nb = 0;    // workgroups of that post-smoother (its partials)
   hipStream_t stream = nullptr;
@@ -157,7 +155,6 @@ struct sp_ctx {
   int tail_level = 0;
   sp::Level<float> lf[sp::kMaxLevels];
   sp::Level<double> ld[sp::kMaxLevels];
-  void* mg_desc = nullptr;  // device copy of the level table for the tail kernel
 
   // GFM stale-beta machinery
   int32_t* stale_list = nullptr;  // (cell, face, kind) triples
@@ -237,6 +234,8 @@ sp_status assemble(sp_ctx* c, const sp_inputs& in, int64_t* stale_count);
 
 // ---- solver (sp_solver.hip) ----
 sp_status mg_setup(sp_ctx* c);
+// Chooses c->tail_level for the allocated levels.
+void mg_tail_level(sp_ctx* c, bool fp32);
 sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool check_true,
                 bool resume);
 sp_status refine(sp_ctx* c, double tol, double* rmax, int* iters);

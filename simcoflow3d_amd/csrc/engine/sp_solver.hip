@@ -18,8 +18,8 @@
 // (restriction = sum over children, prolongation = injection), coarse face
 // coefficients = scale * sum of the fine face coefficients they cover (the
 // Galerkin product for these transfers, scaled), red-black Gauss-Seidel
-// (pre: red,black; post: black,red -- a symmetric V-cycle).  Levels holding
-// at most kTailCells cells run in one single-workgroup kernel.
+// (pre: red,black; post: black,red -- a symmetric V-cycle).  The last levels,
+// of up to about 4096 cells, run in one single-workgroup kernel.
 //
 // Grid kernels run one cell per thread on 64x4 workgroups whose order is
 // remapped so that each XCD owns a contiguous slab (stencil halos stay in one
@@ -178,277 +178,291 @@ __global__ void __launch_bounds__(256) k_prolong(LevelView<T> F, LevelView<T> C,
 
 // ---- single-workgroup V-cycle over the small levels ----
 
-// ---- coarse levels in one workgroup, resident in LDS ----
-
-// One tail level in LDS: couplings, diagonal and its reciprocal, b and x.
-template <typename T>
-struct TailLevel {
-  int nx, ny, nz;
-  T *cx, *cy, *cz, *d, *rd, *b, *x;
-};
-constexpr int kTailArrays = 7;
+// The last levels of the V-cycle in one workgroup.  Every cell belongs to one
+// thread for the whole launch: couplings, b and 1/d in registers, x in LDS
+// (one array per level with a border of zeros, so a neighbour read needs no
+// test).  Threads own i pairs, one red and one black cell: two pairs per
+// thread on the first level, one on one of the others.  All levels are loaded
+// at once.
+//
+// The time is a chain of about forty barrier-separated steps on one CU, so
+// what counts is the instructions and LDS accesses of a step.  With the
+// couplings in LDS too, cell indices formed in every step and the level table
+// read from global memory two levels (8^3 and 4^3) took 22 us a cycle, and a
+// 16^3 level was better off in legs of 9 us (FP32) each; here the three levels
+// take 21 us in FP32 and 29 in FP64 (event times, 5 us of them the launch).
+constexpr int kTailThreads = 1024, kTailLevels = 8;
 
 template <typename T>
 struct TailArgs {
-  int first, last;  // levels [first, last)
-  int pre, post, coarse_sweeps, singular, has_e;
-  T omega, omega_c;  // over-relaxation of the Gauss-Seidel updates (level 0, coarser)
-  const LevelView<T>* lv;   // the levels in global memory
-  T* x;                     // x of the first tail level
-  int off[kMaxLevels];      // element offset of each tail level in LDS
+  int n;  // levels
+  int pre, post, coarse_sweeps, singular;
+  T omega[kTailLevels];  // over-relaxation of the Gauss-Seidel updates
+  int nx[kTailLevels], ny[kTailLevels], nz[kTailLevels];
+  int first[kTailLevels];           // first thread of a level (levels 1 and up)
+  int xo[kTailLevels], ro[kTailLevels];  // LDS offsets: x with its border, residual
+  const T *cx[kTailLevels], *cy[kTailLevels], *cz[kTailLevels], *e[kTailLevels];
+  const T* b;
+  T* x;
 };
 
-template <typename T>
-__device__ inline TailLevel<T> tail_level(T* lds, const TailArgs<T>& A, int l) {
-  const LevelView<T>& G = A.lv[l];
-  const int n = G.nx * G.ny * G.nz;
-  T* base = lds + A.off[l];
-  return TailLevel<T>{G.nx, G.ny, G.nz, base, base + n, base + 2 * n, base + 3 * n,
-                      base + 4 * n, base + 5 * n, base + 6 * n};
-}
+// Threads that a level's pairs take, in whole waves.
+inline int tail_threads(int nx, int ny, int nz) { return ((nx + 1) / 2 * ny * nz + 63) / 64 * 64; }
 
-// (i, j, k) of cell n.  Tail levels hold far fewer than 2^24 cells, so the
-// quotients come from a float reciprocal, corrected by one step (the float
-// estimate is within 1 of the integer quotient).
-struct Ijk {
-  int i, j, k;
-};
+// n / d for n and d below 2^23: the float estimate is within 1 of the quotient.
 __device__ inline unsigned small_div(unsigned n, unsigned d) {
   unsigned q = (unsigned)((float)n * __builtin_amdgcn_rcpf((float)d));
   if (q * d > n) --q;
   else if ((q + 1) * d <= n) ++q;
   return q;
 }
-__device__ inline Ijk ijk_of(unsigned n, unsigned nx, unsigned nxy) {
-  const unsigned k = small_div(n, nxy), r = n - k * nxy, j = small_div(r, nx);
-  return Ijk{(int)(r - j * nx), (int)j, (int)k};
-}
 
-template <typename T>
-__device__ inline T tail_offdiag(const TailLevel<T>& L, int i, int j, int k, int n) {
-  const int sy = L.nx, sz = L.nx * L.ny;
-  T s = T(0);
-  if (i > 0) s += L.cx[n - 1] * L.x[n - 1];
-  if (j > 0) s += L.cy[n - sy] * L.x[n - sy];
-  if (k > 0) s += L.cz[n - sz] * L.x[n - sz];
-  if (i < L.nx - 1) s += L.cx[n] * L.x[n + 1];
-  if (j < L.ny - 1) s += L.cy[n] * L.x[n + sy];
-  if (k < L.nz - 1) s += L.cz[n] * L.x[n + sz];
-  return s;
-}
+// Cells 2a and 2a + 1 of one row; [0] the red one (i + j + k even), [1] the
+// black one.  The second cell of a pair cut by an odd nx has 1/d = 0 and lies
+// on the LDS border, where it writes 0.
+template <typename T, bool HAS_E>
+struct TailPair {
+  T cw[2], ce[2], cs[2], cn[2], cb[2], ct[2], b[2], rd[2];
+  T d[HAS_E ? 2 : 1];  // the diagonal, only where the couplings do not add up to it
+  int at[2];           // x in LDS
+  int m;               // cell index of cell 2a in the level
+  int up;              // x of the parent cell in LDS
+  bool any, hi, odd;   // the pair, its second cell exist; red is the second cell
 
-// The threads that work on a tail level: the whole workgroup, or wave 0
-// alone on the smallest levels, which then need no workgroup barrier (one
-// wave's LDS operations complete in issue order; the fences keep the
-// compiler from moving LDS accesses across the step boundary).
-template <bool WAVE>
-struct TailTeam {
-  __device__ static unsigned id() { return WAVE ? (threadIdx.x & 63u) : threadIdx.x; }
-  __device__ static unsigned size() { return WAVE ? 64u : blockDim.x; }
-  __device__ static void sync() {
-    if (WAVE) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-      __syncthreads();
-    }
+  __device__ inline T diag(int q) const {
+    if (HAS_E) return d[HAS_E ? q : 0];
+    T v = cw[q] + cs[q];
+    v = v + cb[q];
+    v = v + ce[q];
+    v = v + cn[q];
+    return v + ct[q];
+  }
+  // cell index of q, and whether the cell exists
+  __device__ inline int cell(int q) const { return m + ((q == 0) == odd ? 1 : 0); }
+  __device__ inline bool exists(int q) const { return any && (hi || (q == 0) != odd); }
+  // sum of the couplings times the neighbours' x
+  __device__ inline T offdiag(int q, const T* xs, int py, int pz) const {
+    const T* x = xs + at[q];
+    T s = cw[q] * x[-1];
+    s += ce[q] * x[1];
+    s += cs[q] * x[-py];
+    s += cn[q] * x[py];
+    s += cb[q] * x[-pz];
+    s += ct[q] * x[pz];
+    return s;
   }
 };
-constexpr int kTailWaveCells = 64;  // levels this small run on one wave
 
-// One colour of Gauss-Seidel (one thread per cell pair along i); zero_init:
-// x starts at 0 and the other colour is written as 0.  FP32 multiplies by
-// 1/d, FP64 divides by d, as the other smoothers do.
-template <bool WAVE, typename T>
-__device__ void tail_gs(const TailLevel<T>& L, int color, int zero_init, T omega) {
-  using G = TailTeam<WAVE>;
-  const unsigned nxh = (unsigned)(L.nx + 1) / 2, nxy = nxh * (unsigned)L.ny;
-  const unsigned half = nxy * (unsigned)L.nz;
-  for (unsigned t = G::id(); t < half; t += G::size()) {
-    const Ijk q = ijk_of(t, nxh, nxy);
-    const int par = (q.j + q.k + color) & 1;
-    const int i = 2 * q.i + par;
-    const int row = L.nx * (q.j + L.ny * q.k);
-    if (zero_init) {
-      const int io = 2 * q.i + (par ^ 1);
-      if (io < L.nx) L.x[row + io] = T(0);
+template <typename T, bool HAS_E>
+__device__ inline void tail_load(TailPair<T, HAS_E>& P, const TailArgs<T>& A, int l, int t) {
+  const int nx = A.nx[l], ny = A.ny[l], nz = A.nz[l], nxh = (nx + 1) >> 1;
+  P.any = t < nxh * ny * nz;
+  const unsigned tt = P.any ? (unsigned)t : 0u, jk = small_div(tt, nxh), a = tt - jk * nxh;
+  const int k = (int)small_div(jk, ny), j = (int)jk - k * ny;
+  const int py = nx + 2, pz = py * (ny + 2);
+  P.odd = ((j + k) & 1) != 0;
+  P.hi = 2 * (int)a + 1 < nx;
+  P.m = 2 * (int)a + nx * (j + ny * k);
+  // the parent: cell a of row j / 2, plane k / 2 of the next level
+  if (l + 1 < A.n)
+    P.up = A.xo[l + 1] + (int)a + 1 +
+           (A.nx[l + 1] + 2) * ((j >> 1) + 1 + (A.ny[l + 1] + 2) * ((k >> 1) + 1));
+  const T *cx = A.cx[l], *cy = A.cy[l], *cz = A.cz[l], *e = A.e[l];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int second = (q == 0) == P.odd ? 1 : 0, i = 2 * (int)a + second;
+    const bool in = P.exists(q);
+    P.at[q] = A.xo[l] + i + 1 + py * (j + 1) + pz * (k + 1);
+    const int m = in ? P.m + second : P.m;  // a cell that exists
+    const T cw = cx[i > 0 && in ? m - 1 : m], cs = cy[j > 0 ? m - nx : m],
+            cb = cz[k > 0 ? m - nx * ny : m], ce = cx[m], cn = cy[m], ct = cz[m];
+    const T b = l == 0 ? A.b[m] : T(0);
+    // a cell that does not exist has no couplings
+    P.cw[q] = in && i > 0 ? cw : T(0);
+    P.cs[q] = in && j > 0 ? cs : T(0);
+    P.cb[q] = in && k > 0 ? cb : T(0);
+    P.ce[q] = in ? ce : T(0);
+    P.cn[q] = in ? cn : T(0);
+    P.ct[q] = in ? ct : T(0);
+    P.b[q] = in ? b : T(0);
+    // same order as the other kernels: W, S, B, E, N, T, then e
+    T d = P.cw[q] + P.cs[q];
+    d = d + P.cb[q];
+    d = d + P.ce[q];
+    d = d + P.cn[q];
+    d = d + P.ct[q];
+    if (HAS_E) {
+      d = d + (in ? e[m] : T(0));
+      P.d[HAS_E ? q : 0] = d;
     }
-    if (i >= L.nx) continue;
-    const int n = row + i;
-    const T d = L.d[n];
-    if (!(d > T(0))) {
-      if (zero_init) L.x[n] = T(0);
-      continue;
-    }
-    T s = L.b[n];
-    if (!zero_init) s += tail_offdiag(L, i, q.j, q.k, n);
-    const T v = sizeof(T) == 4 ? s * L.rd[n] : s / d;
-    const T x0 = zero_init ? T(0) : L.x[n];
-    L.x[n] = x0 + omega * (v - x0);
+    P.rd[q] = d > T(0) ? T(1) / d : T(0);
   }
-  G::sync();
 }
 
-// v -= mean of v over the cells with d > 0
-template <bool WAVE, typename T>
-__device__ void tail_project_mean(const TailLevel<T>& L, T* v) {
-  using G = TailTeam<WAVE>;
-  __shared__ double red[2][16];
-  double s = 0.0, c = 0.0;
-  const int nn = L.nx * L.ny * L.nz;
-  for (int n = (int)G::id(); n < nn; n += (int)G::size()) {
-    if (L.d[n] > T(0)) { s += (double)v[n]; c += 1.0; }
+// The workgroup's state.  TOP: the first level (two pairs of every thread),
+// otherwise level l (one pair of the threads with mine == l); the two are told
+// apart at compile time so that the pairs stay in registers.
+template <typename T, bool HAS_E>
+struct Tail {
+  using Pair = TailPair<T, HAS_E>;
+  const TailArgs<T>& A;
+  T* xs;
+  double (*red)[kTailThreads / 64];
+  Pair big[2], small;
+  int t, mine;
+
+  template <bool TOP, typename F>
+  __device__ __forceinline__ void own(int l, F f) {
+    if constexpr (TOP) {
+      if (big[0].any) f(big[0]);
+      if (big[1].any) f(big[1]);
+    } else if (mine == l && small.any) {
+      f(small);
+    }
   }
-  s = wave_sum(s);
-  c = wave_sum(c);
-  double ts = 0.0, tc = 0.0;
-  if (WAVE) {
-    ts = __shfl(s, 0, 64);
-    tc = __shfl(c, 0, 64);
-  } else {
-    if ((threadIdx.x & 63) == 0) { red[0][threadIdx.x >> 6] = s; red[1][threadIdx.x >> 6] = c; }
+  template <bool TOP, int Q>
+  __device__ __forceinline__ void sweep(int l, bool zero = false) {
+    const int py = A.nx[l] + 2, pz = py * (A.ny[l] + 2);
+    const T om = A.omega[l];
+    T* x = xs;
+    own<TOP>(l, [=](Pair& P) __attribute__((always_inline)) {
+      // 1/d = 0 keeps cells without couplings at 0
+      if (zero) {
+        x[P.at[Q]] = om * (P.b[Q] * P.rd[Q]);
+      } else {
+        const T x0 = x[P.at[Q]];
+        x[P.at[Q]] = x0 + om * ((P.b[Q] + P.offdiag(Q, x, py, pz)) * P.rd[Q] - x0);
+      }
+    });
     __syncthreads();
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) { ts += red[0][w]; tc += red[1][w]; }
   }
-  const T mean = tc > 0 ? (T)(ts / tc) : T(0);
-  G::sync();
-  for (int n = (int)G::id(); n < nn; n += (int)G::size()) {
-    if (L.d[n] > T(0)) v[n] -= mean;
-  }
-  G::sync();
-}
-
-// coarse b = sum over the 2x2x2 children of the fine residual
-template <bool WAVE, typename T>
-__device__ void tail_restrict(const TailLevel<T>& F, const TailLevel<T>& C) {
-  using G = TailTeam<WAVE>;
-  const unsigned nxy = (unsigned)C.nx * C.ny, nc = nxy * (unsigned)C.nz;
-  for (unsigned t = G::id(); t < nc; t += G::size()) {
-    const Ijk q = ijk_of(t, (unsigned)C.nx, nxy);
-    T s = T(0);
-    for (int cc = 0; cc < 2; ++cc)
-      for (int bb = 0; bb < 2; ++bb)
-        for (int aa = 0; aa < 2; ++aa) {
-          const int fi = 2 * q.i + aa, fj = 2 * q.j + bb, fk = 2 * q.k + cc;
-          if (fi >= F.nx || fj >= F.ny || fk >= F.nz) continue;
-          const int m = fi + F.nx * (fj + F.ny * fk);
-          const T d = F.d[m];
-          if (d > T(0)) s += F.b[m] - (d * F.x[m] - tail_offdiag(F, fi, fj, fk, m));
+  // v -= mean of v over the cells with d > 0 (v: b or x of the last level)
+  template <bool TOP, bool OF_X>
+  __device__ __forceinline__ void project_mean(int l) {
+    double s = 0.0, c = 0.0;
+    T* x = xs;
+    own<TOP>(l, [&](Pair& P) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (P.rd[q] > T(0)) {
+          s += (double)(OF_X ? x[P.at[q]] : P.b[q]);
+          c += 1.0;
         }
-    C.b[t] = s;
+    });
+    s = wave_sum(s);
+    c = wave_sum(c);
+    if ((t & 63) == 0) { red[0][t >> 6] = s; red[1][t >> 6] = c; }
+    __syncthreads();
+    double ts = 0.0, tc = 0.0;
+#pragma unroll
+    for (int w = 0; w < kTailThreads / 64; ++w) { ts += red[0][w]; tc += red[1][w]; }
+    const T mean = tc > 0 ? (T)(ts / tc) : T(0);
+    own<TOP>(l, [=](Pair& P) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (P.rd[q] > T(0)) {
+          if (OF_X) x[P.at[q]] -= mean;
+          else P.b[q] -= mean;
+        }
+    });
+    __syncthreads();
   }
-  G::sync();
-}
-
-template <bool WAVE, typename T>
-__device__ void tail_prolong(const TailLevel<T>& F, const TailLevel<T>& C) {
-  using G = TailTeam<WAVE>;
-  const unsigned nxy = (unsigned)F.nx * F.ny, nf = nxy * (unsigned)F.nz;
-  for (unsigned m = G::id(); m < nf; m += G::size()) {
-    const Ijk q = ijk_of(m, (unsigned)F.nx, nxy);
-    if (F.d[m] > T(0))
-      F.x[m] += C.x[(q.i >> 1) + C.nx * ((q.j >> 1) + C.ny * (q.k >> 1))];
+  // pre-smoothing of level l and coarse b = sum over the 2x2x2 children of
+  // the fine residual
+  template <bool TOP>
+  __device__ __forceinline__ void down(int l) {
+    sweep<TOP, 0>(l, true);
+    sweep<TOP, 1>(l);
+    for (int s = 1; s < A.pre; ++s) { sweep<TOP, 0>(l); sweep<TOP, 1>(l); }
+    T* x = xs;
+    T* r = xs + A.ro[l];
+    const int nx = A.nx[l], ny = A.ny[l], nz = A.nz[l], py = nx + 2, pz = py * (ny + 2);
+    // one value per pair, at the pair's first cell: its two cells are siblings
+    own<TOP>(l, [=](Pair& P) __attribute__((always_inline)) {
+      T v = T(0);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const T w = P.b[q] - (P.diag(q) * x[P.at[q]] - P.offdiag(q, x, py, pz));
+        v += P.rd[q] > T(0) ? w : T(0);
+      }
+      r[P.m] = v;
+    });
+    __syncthreads();
+    if (mine == l + 1 && small.any) {
+      const int cnx = A.nx[l + 1], cny = A.ny[l + 1];
+      // (i, j, k) of the pair's first cell; i is even
+      const unsigned jk = small_div((unsigned)small.m, (unsigned)cnx);
+      const int i = small.m - (int)jk * cnx, k = (int)small_div(jk, (unsigned)cny),
+                j = (int)jk - k * cny;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int ci = i + ((q == 0) == small.odd ? 1 : 0);
+        T s = T(0);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const int fj = 2 * j + (w & 1), fk = 2 * k + (w >> 1);
+          const bool in = 2 * ci < nx && fj < ny && fk < nz;
+          const T v = r[in ? 2 * ci + nx * (fj + ny * fk) : 0];
+          s += in ? v : T(0);
+        }
+        small.b[q] = s;
+      }
+    }
   }
-  G::sync();
-}
+  template <bool TOP>
+  __device__ __forceinline__ void coarsest(int l) {
+    if (A.singular) project_mean<TOP, false>(l);
+    sweep<TOP, 0>(l, true);
+    sweep<TOP, 1>(l);
+    for (int s = 1; s < A.coarse_sweeps; ++s) { sweep<TOP, 0>(l); sweep<TOP, 1>(l); }
+    for (int s = 0; s < A.coarse_sweeps; ++s) { sweep<TOP, 1>(l); sweep<TOP, 0>(l); }
+    if (A.singular) project_mean<TOP, true>(l);
+  }
+  // correction from level l + 1 and post-smoothing of level l
+  template <bool TOP>
+  __device__ __forceinline__ void up(int l) {
+    T* x = xs;
+    own<TOP>(l, [=](Pair& P) __attribute__((always_inline)) {
+      const T v = x[P.up];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (P.rd[q] > T(0)) x[P.at[q]] += v;
+    });
+    __syncthreads();
+    for (int s = 0; s < A.post; ++s) { sweep<TOP, 1>(l); sweep<TOP, 0>(l); }
+  }
+};
 
-template <bool WAVE, typename T>
-__device__ void tail_pre(T* lds, const TailArgs<T>& A, int l) {
-  const TailLevel<T> F = tail_level(lds, A, l);
-  const T om = l == 0 ? A.omega : A.omega_c;
-  tail_gs<WAVE>(F, 0, 1, om);
-  tail_gs<WAVE>(F, 1, 0, om);
-  for (int s = 1; s < A.pre; ++s) { tail_gs<WAVE>(F, 0, 0, om); tail_gs<WAVE>(F, 1, 0, om); }
-  tail_restrict<WAVE>(F, tail_level(lds, A, l + 1));
-}
-
-template <bool WAVE, typename T>
-__device__ void tail_coarsest(T* lds, const TailArgs<T>& A) {
-  const TailLevel<T> C = tail_level(lds, A, A.last - 1);
-  const T om = A.last - 1 == 0 ? A.omega : A.omega_c;
-  if (A.singular) tail_project_mean<WAVE>(C, C.b);
-  tail_gs<WAVE>(C, 0, 1, om);
-  tail_gs<WAVE>(C, 1, 0, om);
-  for (int s = 1; s < A.coarse_sweeps; ++s) { tail_gs<WAVE>(C, 0, 0, om); tail_gs<WAVE>(C, 1, 0, om); }
-  for (int s = 0; s < A.coarse_sweeps; ++s) { tail_gs<WAVE>(C, 1, 0, om); tail_gs<WAVE>(C, 0, 0, om); }
-  if (A.singular) tail_project_mean<WAVE>(C, C.x);
-}
-
-template <bool WAVE, typename T>
-__device__ void tail_post(T* lds, const TailArgs<T>& A, int l) {
-  const TailLevel<T> F = tail_level(lds, A, l);
-  const T om = l == 0 ? A.omega : A.omega_c;
-  tail_prolong<WAVE>(F, tail_level(lds, A, l + 1));
-  for (int s = 0; s < A.post; ++s) { tail_gs<WAVE>(F, 1, 0, om); tail_gs<WAVE>(F, 0, 0, om); }
-}
-
-// The coarse levels of the V-cycle in one workgroup, resident in LDS: the
-// couplings of every tail level and the right-hand side of the first are
-// copied in (the diagonal and 1/d are formed once), the whole sub-cycle
-// runs on LDS, and x of the first tail level is written back for the
-// prolongation above it.
-template <typename T>
-__global__ void __launch_bounds__(1024) k_tail(TailArgs<T> A, const Scalars* S) {
+template <typename T, bool HAS_E>
+__global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A, const Scalars* S) {
   if (S->done) return;
   __shared__ double lds_raw[kTailLdsBytes / sizeof(double)];
-  T* lds = reinterpret_cast<T*>(lds_raw);
-  const int L = A.last;
-  for (int l = A.first; l < L; ++l) {
-    const LevelView<T> G = A.lv[l];
-    const TailLevel<T> V = tail_level(lds, A, l);
-    const int n = G.nx * G.ny * G.nz;
-    for (int q = threadIdx.x; q < n; q += blockDim.x) {
-      V.cx[q] = G.cx[q];
-      V.cy[q] = G.cy[q];
-      V.cz[q] = G.cz[q];
-      V.d[q] = A.has_e ? G.e[q] : T(0);  // diagonal-only term, completed below
-      if (l == A.first) V.b[q] = G.b[q];
-    }
-  }
+  __shared__ double red[2][kTailThreads / 64];
+  Tail<T, HAS_E> W{A, reinterpret_cast<T*>(lds_raw), red, {}, {}, (int)threadIdx.x, 0};
+  tail_load(W.big[0], A, 0, W.t);
+  tail_load(W.big[1], A, 0, W.t + kTailThreads);
+  for (int l = 1; l < A.n; ++l)
+    if (W.t >= A.first[l]) W.mine = l;
+  W.small.any = false;
+  if (W.mine) tail_load(W.small, A, W.mine, W.t - A.first[W.mine]);
+  // the x arrays lie before the residuals
+  for (int q = W.t; q < A.ro[0]; q += kTailThreads) W.xs[q] = T(0);
   __syncthreads();
-  for (int l = A.first; l < L; ++l) {
-    const TailLevel<T> V = tail_level(lds, A, l);
-    const unsigned nxy = (unsigned)V.nx * V.ny, n = nxy * (unsigned)V.nz;
-    for (unsigned m = threadIdx.x; m < n; m += blockDim.x) {
-      const Ijk q = ijk_of(m, (unsigned)V.nx, nxy);
-      // same order as the other kernels: W, S, B, E, N, T, then e
-      T d = q.i > 0 ? V.cx[m - 1] : T(0);
-      d = d + (q.j > 0 ? V.cy[m - V.nx] : T(0));
-      d = d + (q.k > 0 ? V.cz[m - nxy] : T(0));
-      d = d + V.cx[m];
-      d = d + V.cy[m];
-      d = d + V.cz[m];
-      d = d + V.d[m];
-      V.d[m] = d;
-      V.rd[m] = d > T(0) ? T(1) / d : T(0);
-    }
-  }
-  __syncthreads();
-  // levels [first, lw) on the whole workgroup, [lw, L) on wave 0 alone
-  int lw = L;
-  for (int l = A.first; l < L; ++l) {
-    const LevelView<T>& G = A.lv[l];
-    if (G.nx * G.ny * G.nz <= kTailWaveCells) { lw = l; break; }
-  }
-  for (int l = A.first; l < lw && l < L - 1; ++l) tail_pre<false>(lds, A, l);
-  if (lw >= L) {
-    tail_coarsest<false>(lds, A);
+  const int last = A.n - 1;
+  if (last == 0) {
+    W.template coarsest<true>(0);
   } else {
-    if (threadIdx.x < 64) {
-      for (int l = lw; l < L - 1; ++l) tail_pre<true>(lds, A, l);
-      tail_coarsest<true>(lds, A);
-      for (int l = L - 2; l >= lw; --l) tail_post<true>(lds, A, l);
-    }
-    __syncthreads();
+    W.template down<true>(0);
+    for (int l = 1; l < last; ++l) W.template down<false>(l);
+    W.template coarsest<false>(last);
+    for (int l = last - 1; l > 0; --l) W.template up<false>(l);
+    W.template up<true>(0);
   }
-  for (int l = (lw >= L ? L - 2 : lw - 1); l >= A.first; --l) tail_post<false>(lds, A, l);
-  {
-    const LevelView<T> G = A.lv[A.first];
-    const TailLevel<T> V = tail_level(lds, A, A.first);
-    const int n = G.nx * G.ny * G.nz;
-    for (int q = threadIdx.x; q < n; q += blockDim.x) A.x[q] = V.x[q];
-  }
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (W.big[p].exists(q)) A.x[W.big[p].cell(q)] = W.xs[W.big[p].at[q]];
 }
 
 template <typename T>
@@ -1106,25 +1120,36 @@ void vcycle(sp_ctx* c, Level<T>* lv) {
     for (int s = 1; s < cs; ++s) { launch_gs(c, lv[Lc], 0, 0, fine); launch_gs(c, lv[Lc], 1, 0, fine); }
     for (int s = 0; s < cs; ++s) { launch_gs(c, lv[Lc], 1, 0, fine); launch_gs(c, lv[Lc], 0, 0, fine); }
   } else {
-    TailArgs<T> A;
-    A.first = Lt;
-    A.last = L;
+    TailArgs<T> A{};
+    A.n = L - Lt;
     A.pre = pre;
     A.post = post;
     A.coarse_sweeps = std::max(1, c->prm.mg_coarse_sweeps);
-    A.omega = (T)c->prm.mg_omega;
-    A.omega_c = (T)c->prm.mg_omega_coarse;
     A.singular = c->S_host->singular;
-    A.has_e = lv[Lt].e ? 1 : 0;
-    A.lv = reinterpret_cast<const LevelView<T>*>(c->mg_desc);
+    A.b = lv[Lt].b;
     A.x = lv[Lt].x;
-    int64_t off = 0;
-    for (int l = 0; l < kMaxLevels; ++l) {
-      A.off[l] = (int)off;
-      if (l >= Lt && l < L) off += lv[l].n * kTailArrays;
+    int off = 0, thread = 0;
+    for (int q = 0; q < A.n; ++q) {
+      const Level<T>& G = lv[Lt + q];
+      A.omega[q] = (T)(Lt + q == 0 ? c->prm.mg_omega : c->prm.mg_omega_coarse);
+      A.nx[q] = G.nx; A.ny[q] = G.ny; A.nz[q] = G.nz;
+      A.cx[q] = G.cx; A.cy[q] = G.cy; A.cz[q] = G.cz; A.e[q] = G.e;
+      A.xo[q] = off;
+      off += (G.nx + 2) * (G.ny + 2) * (G.nz + 2);
+      A.first[q] = thread;
+      if (q > 0) thread += tail_threads(G.nx, G.ny, G.nz);
+    }
+    for (int q = 0; q < A.n; ++q) {
+      A.ro[q] = off;
+      off += (int)lv[Lt + q].n;
     }
     timer_begin(c, "mg_tail", 0, &slot);
-    hipLaunchKernelGGL(k_tail<T>, dim3(1), dim3(1024), 0, c->stream, A, (const Scalars*)c->S);
+    if (lv[Lt].e)
+      hipLaunchKernelGGL((k_tail<T, true>), dim3(1), dim3(kTailThreads), 0, c->stream, A,
+                         (const Scalars*)c->S);
+    else
+      hipLaunchKernelGGL((k_tail<T, false>), dim3(1), dim3(kTailThreads), 0, c->stream, A,
+                         (const Scalars*)c->S);
     timer_end(c, slot);
   }
   for (int l = Lp - 1; l >= 0; --l) {
@@ -1166,23 +1191,36 @@ sp_status setup_levels(sp_ctx* c, Level<T>* lv) {
                        view_of(lv[l - 1]), view_of(C), C.cx, C.cy, C.cz, C.e,
                        (T)c->prm.mg_coarse_scale);
   }
-  // level table for the tail kernel: it changes only with the buffers and
-  // with the presence of diagonal-only terms
-  if (c->desc_state != (c->has_e ? 1 : 0)) {
-    std::vector<LevelView<T>> desc(kMaxLevels);
-    for (int l = 0; l < L; ++l) desc[l] = view_of(lv[l]);
-    hipError_t e = hipMemcpyAsync(c->mg_desc, desc.data(), sizeof(LevelView<T>) * kMaxLevels,
-                                  hipMemcpyHostToDevice, c->stream);
-    if (e != hipSuccess) return hip_check(c, e, "hipMemcpyAsync(mg_desc)");
-    // the host table must stay valid until the copy has been consumed
-    e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) return hip_check(c, e, "mg setup");
-    c->desc_state = c->has_e ? 1 : 0;
-  }
   return SP_OK;
 }
 
 }  // namespace
+
+// The first level of the tail kernel (c->tail_level): the levels from it on
+// fit its threads (two pairs each on the first level, one on the others) and
+// LDS.  c->levels when not even the coarsest level does (a hierarchy cut short
+// by mg_levels, or a large grid that cannot coarsen): the V-cycle then smooths
+// the coarsest level in global memory.
+template <typename T>
+static int first_tail_level(const Level<T>* lv, int levels) {
+  int best = levels;
+  for (int l = levels - 1; l >= 0 && levels - l <= kTailLevels; --l) {
+    int64_t lds = 0, threads = 0;
+    for (int q = l; q < levels; ++q) {
+      lds += (int64_t)sizeof(T) *
+             ((int64_t)(lv[q].nx + 2) * (lv[q].ny + 2) * (lv[q].nz + 2) + lv[q].n);
+      if (q > l && lv[q].n <= 4 * kTailThreads) threads += tail_threads(lv[q].nx, lv[q].ny, lv[q].nz);
+    }
+    const int64_t pairs = (int64_t)((lv[l].nx + 1) / 2) * lv[l].ny * lv[l].nz;
+    if (pairs > 2 * kTailThreads || threads > kTailThreads || lds > kTailLdsBytes) break;
+    best = l;
+  }
+  return best;
+}
+
+void mg_tail_level(sp_ctx* c, bool fp32) {
+  c->tail_level = fp32 ? first_tail_level(c->lf, c->levels) : first_tail_level(c->ld, c->levels);
+}
 
 sp_status mg_setup(sp_ctx* c) {
   if (c->prm.precond != SP_PRECOND_MG) return SP_OK;
