@@ -89,14 +89,21 @@ static int auto_levels(int I, int J, int K) {
 // smoother legs 140 -> 125 us and 169 -> 156 us (offsets of 1280, 2304 and
 // 4352 bytes measured the same).
 constexpr size_t kStagger = 256, kStaggers = 16;
+// Every buffer ends in kSlack zero bytes: the smoother legs load up to four
+// cells at once, and the load at the end of a row whose length is no multiple
+// of that reads past it, after the last row up to three elements.
+constexpr size_t kSlack = 64;
 
 template <typename T>
 static sp_status dmalloc(sp_ctx* c, T** p, size_t count) {
   void* v = nullptr;
   const size_t off = kStagger * (c->allocs.size() % kStaggers);
-  hipError_t e = hipMalloc(&v, std::max<size_t>(count, 1) * sizeof(T) + off);
+  const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+  hipError_t e = hipMalloc(&v, off + bytes + kSlack);
   if (e != hipSuccess) { *p = nullptr; return hip_check(c, e, "hipMalloc"); }
   c->allocs.push_back(v);
+  e = hipMemsetAsync(static_cast<char*>(v) + off + bytes, 0, kSlack, c->stream);
+  if (e != hipSuccess) { *p = nullptr; return hip_check(c, e, "hipMemsetAsync"); }
   *p = reinterpret_cast<T*>(static_cast<char*>(v) + off);
   return SP_OK;
 }
@@ -200,7 +207,7 @@ static sp_status ensure_buffers(sp_ctx* c) {
   // often.  One allocation for all of it but the first buffer.
   {
     const int64_t bytes = N * (mixed_mg ? 4 : 8);
-    const size_t step = ((size_t)bytes + 255) / 256 * 256 + kStagger;
+    const size_t step = ((size_t)bytes + kSlack + 255) / 256 * 256 + kStagger;
     c->zdepth = 1;
     for (int more = (int)std::min<int64_t>(kZRing, ((int64_t)8 << 30) / bytes) - 1; more > 0;
          more /= 2) {

@@ -13,9 +13,10 @@ namespace sp {
 // the hardware workgroup id so that each XCD receives one contiguous chunk
 // of the logical grid: neighbouring tiles (and their stencil halos) then
 // share one L2.
+// (A count that is no multiple of 8 gives the first total % 8 XCDs one more.)
 __device__ inline uint32_t xcd_logical_block(uint32_t hw, uint32_t total) {
-  if ((total & 7u) != 0u) return hw;
-  return (hw & 7u) * (total >> 3) + (hw >> 3);
+  const uint32_t x = hw & 7u, rest = total & 7u;
+  return x * (total >> 3) + (x < rest ? x : rest) + (hw >> 3);
 }
 
 // Logical (bx, by, bz) of a 3-D launch after the XCD remap.
@@ -149,6 +150,7 @@ struct RedSite {
 // thread 0 (fixed order: lanes, then waves).
 template <int NT, int NV, unsigned MAXMASK>
 __device__ inline void block_reduce_multi(double (&v)[NV]) {
+  static_assert(NT % 64 == 0, "whole waves");
   __shared__ double sm[NV][NT / 64];
   const int tid = flat_tid();
 #pragma unroll

@@ -34,6 +34,7 @@
 #include "sp_device.h"
 #include "sp_geom.h"
 #include "sp_internal.h"
+#include "sp_smooth_cell.h"
 #include "sp_smooth_fused.h"
 
 namespace sp {
@@ -102,8 +103,7 @@ __global__ void __launch_bounds__(256) k_gs(LevelView<T> L, int color, int zero_
   }
   T s = L.b[n];
   if (!zero_init) s += offdiag_sum(L, i, j, k, n);
-  // same rounding as the fused smoother (FP32: times 1/d, FP64: divided by d),
-  // over-relaxed by omega
+  // FP32 multiplies by the hardware reciprocal; over-relaxed by omega
   const T v = sizeof(T) == 4 ? s * smoother_rcp(d) : s / d;
   const T x0 = zero_init ? T(0) : L.x[n];
   L.x[n] = x0 + omega * (v - x0);
@@ -625,7 +625,7 @@ __global__ void __launch_bounds__(256) k_cg_residual(CgArgs A, int from_zero) {
         const double rr = fabs(rv) / (dxy * dz[cc]);
         v[0] = (rr > v[0] || rr != rr) ? rr : v[0];
         if (!is_finite(rv)) v[1] = 1.0;
-        v[2] += rv;
+        v[2] += A.r32 ? (double)(float)rv : rv;
       }
       A.r[n] = rv;
       if (A.r32) A.r32[n] = (float)rv;
@@ -711,7 +711,9 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_dots_fin(CgArgs A, uint32_t 
 // is a fixed symmetric operator up to its own rounding (pre: red, black,
 // post: black, red, restriction the transpose of the prolongation), so z is
 // orthogonal to the previous residual and beta = rz / rz_old needs no (z,q):
-// the leg does not have to read q.
+// the leg does not have to read q.  (Iteration counts with and without it
+// agree to 2 in 180 on flat grids that need that many, and are equal below
+// 100; k_cg_spmv_fin takes what rounding leaves of (z,q) into the step.)
 __global__ void __launch_bounds__(kFinThreads) k_cg_dots2_fin(CgArgs A, uint32_t nb) {
   Scalars* S = A.S;
   if (S->done) return;
@@ -737,7 +739,7 @@ __global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
   Scalars* S = A.S;
   if (S->done) return;
   const Col3 q = col_of(A.I, A.J, A.K);
-  double v[2] = {0.0, 0.0};  // (z - m, q), sum q
+  double v[3] = {0.0, 0.0, 0.0};  // (z - m, q), sum q, (z - m, q_old)
   if (q.in) {
     const double beta = S->beta, m = S->zshift;
     const int64_t I = A.I, IJ = (int64_t)A.I * A.J;
@@ -777,30 +779,39 @@ __global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
       A.q[n] = qv;
       v[0] += (zc - m) * qv;
       v[1] += qv;
+      v[2] += (zc - m) * qo;
       zm = zc;
       zc = zp;
       czm = cz;
     }
   }
-  block_partials<kTileThreads, 2, 0u>(A.site, v);
+  block_partials<kTileThreads, 3, 0u>(A.site, v);
 }
 
 __global__ void __launch_bounds__(kFinThreads) k_cg_spmv_fin(CgArgs A, uint32_t nb) {
   Scalars* S = A.S;
   if (S->done) return;
-  double t[2];
-  finalize_partials<kFinThreads, 2, 0u>(A.site, nb, t);
+  double t[3];
+  finalize_partials<kFinThreads, 3, 0u>(A.site, nb, t);
   if (flat_tid() == 0) {
-    S->pq = t[0];
+    const double beta = S->beta;
+    // (p, q) of p = (z - m) + beta p_old, also where beta has left p a little
+    // short of A-orthogonal to p_old: alpha then still is the exact minimiser
+    // along p (pq holds the last step's value, beta is 0 in the first)
+    const double pq = t[0] + (beta != 0.0 ? beta * (t[2] + beta * S->pq) : 0.0);
+    S->pq = pq;
     S->qsum = t[1];
-    S->alpha = S->rz / t[0];
+    S->alpha = S->rz / pq;
     S->hist_alpha[A.slot] = S->alpha;
     S->nhist = A.slot + 1;
     if (!is_finite(S->alpha)) { S->nonfinite = 1; S->done = 1; }
   }
 }
 
-// r -= alpha q ; rmax = max |r|/V
+// r -= alpha q ; rmax = max |r|/V, and the sum of r as the V-cycle sees it
+// (rounded to FP32 with an FP32 one): (r, z - m) is formed as (r, z) - m sum r,
+// which is exact in m only with the sum of the very r of (r, z); z may sit on a
+// shift m much larger than its variation.
 __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
   Scalars* S = A.S;
   if (S->done) return;
@@ -818,7 +829,7 @@ __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
       if (A.r32) A.r32[n] = (float)rv;
       const double rr = fabs(rv) / (dxy * A.dzp[c]);
       v[0] = (rr > v[0] || rr != rr) ? rr : v[0];  // a NaN sticks
-      v[1] += rv;
+      v[1] += A.r32 ? (double)(float)rv : rv;
     }
   }
   block_partials<kTileThreads, 2, 1u>(A.site, v);
@@ -986,56 +997,84 @@ void launch_cheb(sp_ctx* c, const Level<T>& L, int m, bool from_zero, bool fine)
     hipMemcpyAsync(L.x, in, sizeof(T) * (size_t)L.n, hipMemcpyDeviceToDevice, c->stream);
 }
 
-// One smoother leg with extended tiles of EX x EY threads; per_cu: how many
-// such workgroups a CU holds at once (registers and LDS).
-template <typename T, int NU, int EX, int EY>
-void launch_fused_tile(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode,
-                       int per_cu) {
-  using Sh = FusedShape<NU, EX, EY>;
+// Grid of a smoother leg, and its k chunk: even (coarse cells never straddle
+// chunks).  A workgroup marches kchunk + 2H planes one after the other, so pick
+// the chunk that minimises rounds-of-workgroups x planes marched.
+template <typename Sh, typename T>
+dim3 leg_grid(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, int per_cu) {
   const int gx = (L.nx + Sh::TX - 1) / Sh::TX, gy = (L.ny + Sh::TY - 1) / Sh::TY;
-  // k chunk: even (coarse cells never straddle chunks).  A workgroup marches
-  // kchunk + 2H planes one after the other, so pick the chunk that minimises
-  // rounds-of-workgroups x planes marched.
-  {
-    const int64_t tiles = (int64_t)gx * gy, slots = (int64_t)std::max(1, c->num_cu) * per_cu;
-    const int kmax = (L.nz + 1) & ~1;
-    int best = kmax;
-    int64_t best_cost = -1;
-    for (int kc = 2; kc <= kmax; kc += 2) {
-      const int64_t blocks = tiles * ((L.nz + kc - 1) / kc);
-      const int64_t cost = ((blocks + slots - 1) / slots) * (kc + 2 * Sh::H);
-      if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = kc; }
-    }
-    A.kchunk = best;
+  const int64_t tiles = (int64_t)gx * gy, slots = (int64_t)std::max(1, c->num_cu) * per_cu;
+  const int kmax = (L.nz + 1) & ~1;
+  int64_t best_cost = -1;
+  for (int kc = 2; kc <= kmax; kc += 2) {
+    const int64_t blocks = tiles * ((L.nz + kc - 1) / kc);
+    const int64_t cost = ((blocks + slots - 1) / slots) * (kc + 2 * Sh::H);
+    if (best_cost < 0 || cost < best_cost) { best_cost = cost; A.kchunk = kc; }
   }
-  const dim3 grd(gx, gy, (L.nz + A.kchunk - 1) / A.kchunk), blk(EX, EY, 1);
-  int slot;
+  const dim3 grd(gx, gy, (L.nz + A.kchunk - 1) / A.kchunk);
   if (A.dots) c->dots_nb = grd.x * grd.y * grd.z;
-  // algorithmic words per cell: pre b + 3 faces -> x (+ coarse b);
-  // post x_pre + 3 faces + b -> x (+ coarse x)
-  const double words = mode == 0 ? 5.0 + 0.125 : 6.0 + 0.125;
-  timer_begin(c, fine ? (mode == 0 ? "mg_pre_fine" : "mg_post_fine")
-                      : (mode == 0 ? "mg_pre_coarse" : "mg_post_coarse"),
-              level_bytes(L, words + (L.e ? 1.0 : 0.0)), &slot);
-  const Scalars* S = c->S;
-#define SP_FUSED_LAUNCH(MODE_, FINE_)                                                         \
-  do {                                                                                        \
-    if (A.e)                                                                                  \
-      hipLaunchKernelGGL((k_smooth_fused<T, NU, MODE_, FINE_, true, EX, EY>), grd, blk, 0,    \
-                         c->stream, A, S);                                                    \
-    else                                                                                      \
-      hipLaunchKernelGGL((k_smooth_fused<T, NU, MODE_, FINE_, false, EX, EY>), grd, blk, 0,   \
-                         c->stream, A, S);                                                    \
+  return grd;
+}
+
+// One smoother leg.  KERNEL(MODE, FINE): the kernel of a form.
+#define SP_LEG(KERNEL)                                                                         \
+  do {                                                                                         \
+    if (mode == 0) hipLaunchKernelGGL((KERNEL(0, false)), grd, blk, 0, c->stream, A, S);       \
+    else if (fine) hipLaunchKernelGGL((KERNEL(1, true)), grd, blk, 0, c->stream, A, S);        \
+    else hipLaunchKernelGGL((KERNEL(1, false)), grd, blk, 0, c->stream, A, S);                 \
   } while (0)
-  if (mode == 0) {
-    if (fine) SP_FUSED_LAUNCH(0, true);
-    else SP_FUSED_LAUNCH(0, false);
-  } else {
-    if (fine) SP_FUSED_LAUNCH(1, true);
-    else SP_FUSED_LAUNCH(1, false);
+
+template <typename T, int NU, bool HAS_E, bool SMALL>
+void launch_march(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode) {
+  using Tile = FusedTile<T, SMALL>;
+  constexpr int Q = Tile::Q, EP = Tile::EP, EY = Tile::EY;
+  const dim3 grd = leg_grid<FusedShape<NU, Q, EP, EY>>(c, L, A, Tile::kPerCu), blk(EP * EY, 1, 1);
+  const Scalars* S = c->S;
+#define SP_K(MODE, FINE) k_smooth_fused<T, NU, Q, MODE, FINE, HAS_E, EP, EY>
+  SP_LEG(SP_K);
+#undef SP_K
+}
+
+template <typename T, int NU, bool HAS_E, int EX, int EY>
+void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode, int per_cu) {
+  const dim3 grd = leg_grid<CellShape<NU, EX, EY>>(c, L, A, per_cu), blk(EX, EY, 1);
+  const Scalars* S = c->S;
+#define SP_K(MODE, FINE) k_smooth_cell<T, NU, MODE, FINE, HAS_E, EX, EY>
+  SP_LEG(SP_K);
+#undef SP_K
+}
+#undef SP_LEG
+
+// FP32: four cells per thread on levels without a diagonal-only term and of
+// more than kCellColumns columns, else one cell per thread.
+template <int NU>
+void launch_leg(sp_ctx* c, const Level<float>& L, FusedArgs<float>& A, bool fine, int mode) {
+  const int64_t cols = (int64_t)L.nx * L.ny;
+  if (!A.e && cols > kCellColumns) {
+    launch_march<float, NU, false, false>(c, L, A, fine, mode);
+    return;
   }
-#undef SP_FUSED_LAUNCH
-  timer_end(c, slot);
+  // a level of at most 32 x 32 columns has two 32 x 16 tiles: its 10-step
+  // marches (2 planes + the 8-plane pipeline) run on 32 CUs.  Small tiles put
+  // a workgroup on every CU (32^3: 10.5 -> 7.8 us per leg); at 64 x 64 they
+  // measured slower than the large ones (13.0 against 11.7 us)
+  if (!fine && cols <= 32 * 32) {
+    if (A.e) launch_cell<float, NU, true, kFEXs, kFEYs>(c, L, A, fine, mode, 4);
+    else launch_cell<float, NU, false, kFEXs, kFEYs>(c, L, A, fine, mode, 4);
+  } else {
+    if (A.e) launch_cell<float, NU, true, kFEX, kFEY>(c, L, A, fine, mode, 1);
+    else launch_cell<float, NU, false, kFEX, kFEY>(c, L, A, fine, mode, 1);
+  }
+}
+template <int NU>
+void launch_leg(sp_ctx* c, const Level<double>& L, FusedArgs<double>& A, bool fine, int mode) {
+  if ((int64_t)L.nx * L.ny <= kSmallColumns) {
+    if (A.e) launch_march<double, NU, true, true>(c, L, A, fine, mode);
+    else launch_march<double, NU, false, true>(c, L, A, fine, mode);
+  } else {
+    if (A.e) launch_march<double, NU, true, false>(c, L, A, fine, mode);
+    else launch_march<double, NU, false, false>(c, L, A, fine, mode);
+  }
 }
 
 template <typename T, int NU>
@@ -1055,14 +1094,15 @@ void launch_fused(sp_ctx* c, Level<T>* lv, int l, int mode) {
     A.dsite = red_site(c, kSiteDots);
   }
   const bool fine = l == 0;
-  // a level of at most 32 x 32 columns has two 32 x 16 tiles: its 10-step
-  // marches (2 planes + the 8-plane pipeline) run on 32 CUs.  Small tiles put
-  // a workgroup on every CU (32^3: 10.5 -> 7.8 us per leg); at 64 x 64 they
-  // measured slower than the large ones (13.0 against 11.7 us)
-  if (!fine && (int64_t)L.nx * L.ny <= 32 * 32)
-    launch_fused_tile<T, NU, kFEXs, kFEYs>(c, L, A, fine, mode, 4);
-  else
-    launch_fused_tile<T, NU, kFEX, kFEY>(c, L, A, fine, mode, 1);
+  int slot;
+  // algorithmic words per cell: pre b + 3 faces -> x (+ coarse b);
+  // post x_pre + 3 faces + b -> x (+ coarse x)
+  const double words = mode == 0 ? 5.0 + 0.125 : 6.0 + 0.125;
+  timer_begin(c, fine ? (mode == 0 ? "mg_pre_fine" : "mg_post_fine")
+                      : (mode == 0 ? "mg_pre_coarse" : "mg_post_coarse"),
+              level_bytes(L, words + (L.e ? 1.0 : 0.0)), &slot);
+  launch_leg<NU>(c, L, A, fine, mode);
+  timer_end(c, slot);
 }
 
 // The V-cycle uses the temporally blocked smoother legs
@@ -1309,10 +1349,9 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
   volatile int32_t* hflag = c->hflags;
   // the finest post-smoother forms the CG dot products when the V-cycle has
   // a fused leg on the finest level (a level above the tail, or above the
-  // coarsest when no level fits the tail) and an FP32 V-cycle (the FP64
-  // smoother has no registers to spare for the extra inputs)
+  // coarsest when no level fits the tail)
   const int legs = c->tail_level < c->levels ? c->tail_level : c->levels - 1;
-  c->fuse_dots = mg && mixed && fused_vcycle(c) && legs > 0;
+  c->fuse_dots = mg && fused_vcycle(c) && legs > 0;
   c->dots_nb = 0;
   hipEvent_t evs[2];
   hipEventCreateWithFlags(&evs[0], hipEventDisableTiming);
