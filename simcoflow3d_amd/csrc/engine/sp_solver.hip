@@ -655,6 +655,9 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_residual_fin(CgArgs A, uint3
   }
 }
 
+// cells per thread of k_cg_spmv and k_cg_update on small grids
+constexpr int kColShort = 4;
+
 // The scalars of the new search direction p = (z - m) + beta p_old.
 __device__ inline void set_direction(Scalars* S, int slot, double m, double rz, double beta) {
   S->zshift = m;
@@ -734,11 +737,11 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_dots2_fin(CgArgs A, uint32_t
 // cells have no couplings and z = 0: q stays 0 there without a mask.  Each
 // thread walks its column keeping z and the z-coupling of planes k-1 / k /
 // k+1 in registers.
-template <typename Z>
+template <typename Z, int KC>
 __global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
   Scalars* S = A.S;
   if (S->done) return;
-  const Col3 q = col_of(A.I, A.J, A.K);
+  const Col3 q = col_of<KC>(A.I, A.J, A.K);
   double v[3] = {0.0, 0.0, 0.0};  // (z - m, q), sum q, (z - m, q_old)
   if (q.in) {
     const double beta = S->beta, m = S->zshift;
@@ -812,10 +815,11 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_spmv_fin(CgArgs A, uint32_t 
 // (rounded to FP32 with an FP32 one): (r, z - m) is formed as (r, z) - m sum r,
 // which is exact in m only with the sum of the very r of (r, z); z may sit on a
 // shift m much larger than its variation.
+template <int KC>
 __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
   Scalars* S = A.S;
   if (S->done) return;
-  const Col3 q = col_of(A.I, A.J, A.K);
+  const Col3 q = col_of<KC>(A.I, A.J, A.K);
   const double alpha = S->alpha;
   double v[2] = {0.0, 0.0};  // max |r|/V, sum r
   if (q.in) {
@@ -1307,6 +1311,17 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
 
   const uint32_t ncol = col_blocks(D.I, D.J, D.K);
   const dim3 cgrd = col_grid(D.I, D.J, D.K);
+  // Cells per thread of k_cg_spmv and k_cg_update: kColK where that puts four
+  // workgroups on every CU, kColShort below, where the 16 planes one after the
+  // other are the time (event times of both kernels: 32^3 13.6 and 9.5 -> 7.6
+  // and 6.9 us, 64^3 17.9 and 12.0 -> 8.7 and 7.5, 97 x 130 x 75 19.5 and 14.3
+  // -> 13.2 and 10.7, 128^3 21.3 and 16.2 -> 19.7 and 14.4; at 160^3, beyond
+  // the limit, 40.4 and 21.7 against 39.4 and 22.8 with four times the partial
+  // sums).
+  const bool shortcol = ncol < 4u * (uint32_t)std::max(1, c->num_cu);
+  const uint32_t nshort = col_blocks_k<kColShort>(D.I, D.J, D.K);
+  const dim3 sgrd = shortcol ? col_grid_k<kColShort>(D.I, D.J, D.K) : cgrd;
+  const uint32_t nsp = shortcol ? nshort : ncol;
   auto launch_col = [&](auto kern, int site, const char* name, double bytes) {
     A.site = red_site(c, site);
     timer_begin(c, name, bytes, &slot);
@@ -1412,16 +1427,27 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
       {
         A.site = red_site(c, kSiteSpmv);
         timer_begin(c, "cg_spmv", NB * (zb + 8 + 24 + eb + 8), &slot);
-        if (A.z32)
-          hipLaunchKernelGGL(k_cg_spmv<float>, cgrd, blk, 0, c->stream, A, (const float*)A.z32);
+        const float* zf = A.z32;
+        const double* zd = A.z64;
+        if (zf && shortcol)
+          hipLaunchKernelGGL((k_cg_spmv<float, kColShort>), sgrd, blk, 0, c->stream, A, zf);
+        else if (zf)
+          hipLaunchKernelGGL((k_cg_spmv<float, kColK>), sgrd, blk, 0, c->stream, A, zf);
+        else if (shortcol)
+          hipLaunchKernelGGL((k_cg_spmv<double, kColShort>), sgrd, blk, 0, c->stream, A, zd);
         else
-          hipLaunchKernelGGL(k_cg_spmv<double>, cgrd, blk, 0, c->stream, A,
-                             (const double*)A.z64);
+          hipLaunchKernelGGL((k_cg_spmv<double, kColK>), sgrd, blk, 0, c->stream, A, zd);
         timer_end(c, slot);
       }
-      finalize(k_cg_spmv_fin, kSiteSpmv, ncol);
-      launch_col(k_cg_update, kSiteUpdate, "cg_update", NB * (8 * 2 + 8 + (A.r32 ? 4 : 0)));
-      finalize(k_cg_update_fin, kSiteUpdate, ncol);
+      finalize(k_cg_spmv_fin, kSiteSpmv, nsp);
+      A.site = red_site(c, kSiteUpdate);
+      timer_begin(c, "cg_update", NB * (8 * 2 + 8 + (A.r32 ? 4 : 0)), &slot);
+      if (shortcol)
+        hipLaunchKernelGGL(k_cg_update<kColShort>, sgrd, blk, 0, c->stream, A);
+      else
+        hipLaunchKernelGGL(k_cg_update<kColK>, sgrd, blk, 0, c->stream, A);
+      timer_end(c, slot);
+      finalize(k_cg_update_fin, kSiteUpdate, nsp);
       hipEventRecord(evs[cur], c->stream);
       ++it;
       ++A.slot;
