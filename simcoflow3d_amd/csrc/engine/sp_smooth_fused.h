@@ -62,21 +62,20 @@ struct FusedArgs {
 
 // The extended tile of a leg (threads along i x rows) and pairs per thread.
 //
-// The leg is bound by the lines it pulls through L2 (its extended tiles, 1.9
-// times the interior) and by the step's instruction stream, about evenly.
+// The leg is bound by the lines it pulls through L2 (its extended tiles, 1.7 to
+// 1.9 times the interior) and by the step's instruction stream, about evenly.
 // FP32: four cells per thread with 16-byte loads (256 VGPRs, two waves per
 // SIMD), a 64 x 16 interior whose rows are whole cache lines; measured at
 // 256^3 with one cell per thread and a 32 x 16 interior 117 (pre) and 140 us
 // (post), with a pair and 56 x 16 120 and 133 us, with this 105 and 116 us
-// (floor at the card's copy rate: 70 and 84 us).  FP64, whose windows do not
-// fit the registers twice: a pair per thread, 32 x 16 interior (256^3: 272 and
-// 274 -> 253 and 256 us).
+// (floor at the card's copy rate: 70 and 84 us; all on one card).  FP64, whose
+// windows do not fit the registers twice: a pair per thread, 32 x 16 interior
+// (256^3: 272 and 274 -> 253 and 256 us).
 //
 // FP64 levels of at most 64 x 64 columns give too few large tiles to put one
 // on every CU, and a march of few steps whose time is the latency of a step:
-// 8 x 8 interior, two waves per workgroup (FP64 leg, pre
-// and post, against the former one-cell kernel: whole solves at 32^3 1642 ->
-// 1257 us, 128^3 4175 -> 3542 us).
+// 8 x 8 interior, two waves per workgroup (against one cell per thread, whole
+// solves at 32^3 1642 -> 1257 us, 128^3 4175 -> 3542 us).
 template <typename T, bool SMALL>
 struct FusedTile {
   static constexpr bool kQuad = sizeof(T) == 4;
