@@ -17,7 +17,7 @@ module simco_proj
   public :: sp_params, sp_inputs, sp_outputs, sp_stats, sp_adj_inputs, sp_adj_outputs, &
             sp_wall_bc, sp_vtr_fields, sp_vtk_fields, sp_solid_body, sp_lvs_grid, sp_clsvof_inputs, sp_clsvof_state, sp_cell_geom, sp_cell_interp, sp_liquid_field, &
             sp_pred_inputs, sp_pred_outputs
-  public :: sp_params_default, sp_create, sp_destroy, sp_set_params, sp_set_grid, &
+  public :: sp_params_default, sp_create, sp_destroy, sp_set_params, sp_set_solver_memory, sp_set_grid, &
             sp_set_grid_1d, sp_project, sp_project_dev, sp_adjoint, sp_adjoint_dev, &
             sp_wall_step, sp_wall_step_dev, sp_write_vtr, sp_write_vtk, sp_interpolate_lvs, sp_clsvof_scheme, sp_grid_preprocess, &
             sp_grid_preprocess_dev, sp_new_cell_face, sp_define_momentum_exchange_cell, &
@@ -257,6 +257,13 @@ module simco_proj
       type(c_ptr), value :: ctx
       type(sp_params), intent(in) :: params
     end function sp_set_params
+
+    ! most device memory (bytes) the solver keeps beyond what it cannot do without
+    integer(c_int) function sp_set_solver_memory(ctx, bytes) bind(C, name="sp_set_solver_memory")
+      import :: c_ptr, c_int, c_int64_t
+      type(c_ptr), value :: ctx
+      integer(c_int64_t), value :: bytes
+    end function sp_set_solver_memory
 
     ! PGrid%dx,dy,dz, UGrid%dx, VGrid%dy, WGrid%dz (Imax x Jmax x Kmax each)
     integer(c_int) function sp_set_grid(ctx, dxp, dyp, dzp, dxu, dyv, dzw) &

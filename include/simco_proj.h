@@ -212,6 +212,17 @@ sp_status sp_destroy(sp_ctx* ctx);
 /* Replace the solver parameters (same grid size). */
 sp_status sp_set_params(sp_ctx* ctx, const sp_params* params);
 
+/* Most device memory, in bytes, that the solver keeps beyond what it cannot do
+ * without: the preconditioned residuals of up to 16 CG steps, from which the
+ * pressure is formed in one pass (4 bytes a cell and step with SP_PREC_MIXED
+ * and multigrid, else 8: 0.9 GiB at 256^3 mixed, 1.9 GiB FP64).  Default
+ * 8 GiB; 0: none, every step then updates the pressure by itself (slower).
+ * At most a sixteenth of the device's free memory is taken, with the first
+ * projection; it is given back when an allocation of any context of the
+ * process finds no room on the device, and with sp_destroy.  Takes effect with
+ * the next projection. */
+sp_status sp_set_solver_memory(sp_ctx* ctx, int64_t bytes);
+
 /* Grid (Mesh.f90:14-18): PGrid%dx,dy,dz and the staggered centre distances
  * UGrid%dx, VGrid%dy, WGrid%dz (Mesh.f90:160-247), as the host's 3-D arrays.
  * The grid must be a tensor product (dx depends on i only, ...). */

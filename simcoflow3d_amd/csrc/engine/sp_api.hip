@@ -99,7 +99,7 @@ static sp_status dmalloc(sp_ctx* c, T** p, size_t count) {
   void* v = nullptr;
   const size_t off = kStagger * (c->allocs.size() % kStaggers);
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-  hipError_t e = hipMalloc(&v, off + bytes + kSlack);
+  hipError_t e = dev_malloc(c, &v, off + bytes + kSlack);
   if (e != hipSuccess) { *p = nullptr; return hip_check(c, e, "hipMalloc"); }
   c->allocs.push_back(v);
   e = hipMemsetAsync(static_cast<char*>(v) + off + bytes, 0, kSlack, c->stream);
@@ -108,7 +108,77 @@ static sp_status dmalloc(sp_ctx* c, T** p, size_t count) {
   return SP_OK;
 }
 
+// The contexts that hold a z ring (never destroyed: a context may outlive the
+// library's static objects).
+struct ZRings {
+  std::mutex mutex;
+  std::vector<sp_ctx*> held;
+};
+static ZRings& zrings() {
+  static ZRings* r = new ZRings;
+  return *r;
+}
+
+// Gives the ring of `o` back; zrings().mutex is held.
+static void zring_free(sp_ctx* o) {
+  std::lock_guard<std::mutex> solve(o->zmutex);
+  hipFree(o->zslab);
+  o->zslab = nullptr;
+  o->zdepth = 1;
+}
+
+static void zring_drop(sp_ctx* c) {
+  ZRings& R = zrings();
+  std::lock_guard<std::mutex> lock(R.mutex);
+  const auto it = std::find(R.held.begin(), R.held.end(), c);
+  if (it == R.held.end()) return;
+  zring_free(c);
+  R.held.erase(it);
+}
+
+hipError_t dev_malloc(sp_ctx* c, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  {
+    ZRings& R = zrings();
+    std::lock_guard<std::mutex> lock(R.mutex);
+    const auto mine = [&](sp_ctx* o) { return o->device == c->device; };
+    if (std::none_of(R.held.begin(), R.held.end(), mine)) return e;
+    for (sp_ctx* o : R.held)
+      if (mine(o)) zring_free(o);
+    R.held.erase(std::remove_if(R.held.begin(), R.held.end(), mine), R.held.end());
+  }
+  return hipMalloc(p, bytes);
+}
+
+// The buffers of the z ring behind the first: as many as zlimit and a part of
+// the device's free memory hold, in one allocation, none when it is refused.
+// A ring that was given back is not taken again before the buffers are made
+// anew.
+static void zring_take(sp_ctx* c) {
+  c->zdue = false;
+  c->zdepth = 1;
+  const bool f32 = c->prm.precision == SP_PREC_MIXED && c->prm.precond == SP_PRECOND_MG;
+  const size_t bytes = (size_t)c->dm.N * (f32 ? 4 : 8);
+  const size_t step = (bytes + 255) / 256 * 256 + kStagger;
+  size_t free = 0, total = 0;
+  if (hipMemGetInfo(&free, &total) != hipSuccess) { (void)hipGetLastError(); return; }
+  const size_t room = std::min<size_t>((size_t)c->zlimit, free / kZRingShare);
+  const int more = (int)std::min<size_t>(kZRing - 1, room / step);
+  if (more < 1) return;
+  void* v = nullptr;
+  if (hipMalloc(&v, kStagger + step * (size_t)more) != hipSuccess) { (void)hipGetLastError(); return; }
+  c->zslab = v;
+  for (int j = 0; j < more; ++j)
+    c->zring[c->zdepth++] = static_cast<char*>(v) + kStagger + step * (size_t)j;
+  ZRings& R = zrings();
+  std::lock_guard<std::mutex> lock(R.mutex);
+  R.held.push_back(c);
+}
+
 static void free_buffers(sp_ctx* c) {
+  zring_drop(c);
   for (void* p : c->allocs) hipFree(p);
   c->allocs.clear();
   c->allocated_for = 0;
@@ -153,8 +223,10 @@ static sp_status ensure_buffers(sp_ctx* c) {
   if (pc != SP_PRECOND_MG) L = 1;
   const int cheb = (c->prm.flags & SP_FLAG_CHEBYSHEV) ? 1 : 0;
   if (c->allocated_for == (size_t)D.N && c->allocated_prec == prec && c->allocated_precond == pc &&
-      c->allocated_levels == L && c->allocated_cheb == cheb)
+      c->allocated_levels == L && c->allocated_cheb == cheb) {
+    if (c->zdue) zring_take(c);
     return SP_OK;
+  }
   free_buffers(c);
   c->levels = L;
   const int64_t N = D.N;
@@ -202,25 +274,7 @@ static sp_status ensure_buffers(sp_ctx* c) {
   if ((s = dmalloc(c, &c->wall_var,
                    8 * ((int64_t)D.J * D.K + (int64_t)D.I * D.K + (int64_t)D.I * D.J))))
     return s;
-  // The z ring: as deep as 8 GiB allow (16 buffers up to 512x512x512 in FP32),
-  // and shallower when the device has no room: a solve then forms x more
-  // often.  One allocation for all of it but the first buffer.
-  {
-    const int64_t bytes = N * (mixed_mg ? 4 : 8);
-    const size_t step = ((size_t)bytes + kSlack + 255) / 256 * 256 + kStagger;
-    c->zdepth = 1;
-    for (int more = (int)std::min<int64_t>(kZRing, ((int64_t)8 << 30) / bytes) - 1; more > 0;
-         more /= 2) {
-      char* z;
-      if (dmalloc(c, &z, step * (size_t)more) != SP_OK) {
-        (void)hipGetLastError();
-        c->last_error.clear();
-        continue;
-      }
-      for (int j = 0; j < more; ++j) c->zring[c->zdepth++] = z + step * (size_t)j;
-      break;
-    }
-  }
+  zring_take(c);
   c->allocated_for = (size_t)N;
   c->allocated_prec = prec;
   c->allocated_precond = pc;
@@ -410,7 +464,7 @@ static sp_status stage(sp_ctx* c, size_t idx, size_t bytes, void** out) {
     if (b.ptr) hipFree(b.ptr);
     b.ptr = nullptr;
     b.bytes = 0;
-    hipError_t e = hipMalloc(&b.ptr, bytes);
+    hipError_t e = dev_malloc(c, &b.ptr, bytes);
     if (e != hipSuccess) return hip_check(c, e, "hipMalloc(stage)");
     b.bytes = bytes;
   }
@@ -490,16 +544,19 @@ sp_status sp_create(sp_ctx** out, const sp_params* params, int device) {
   D.N = (int64_t)D.I * D.J * D.K;
   D.SX = D.I + 2; D.SY = D.J + 2;
   D.Nh = (int64_t)D.SX * D.SY * (D.K + 2);
-  if (hipMalloc(&c->S, sizeof(Scalars)) != hipSuccess ||
+  auto vector = [c](double** p, int n) {
+    return dev_malloc(c, reinterpret_cast<void**>(p), sizeof(double) * (size_t)n);
+  };
+  if (dev_malloc(c, reinterpret_cast<void**>(&c->S), sizeof(Scalars)) != hipSuccess ||
       hipHostMalloc(&c->S_host, sizeof(Scalars), hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&c->hflags, 4 * sizeof(int32_t), hipHostMallocMapped) != hipSuccess ||
       hipHostGetDevicePointer((void**)&c->hflags_dev, c->hflags, 0) != hipSuccess ||
-      hipMalloc(&c->dxp, sizeof(double) * D.I) != hipSuccess ||
-      hipMalloc(&c->dyp, sizeof(double) * D.J) != hipSuccess ||
-      hipMalloc(&c->dzp, sizeof(double) * D.K) != hipSuccess ||
-      hipMalloc(&c->dxu, sizeof(double) * D.I) != hipSuccess ||
-      hipMalloc(&c->dyv, sizeof(double) * D.J) != hipSuccess ||
-      hipMalloc(&c->dzw, sizeof(double) * D.K) != hipSuccess) {
+      vector(&c->dxp, D.I) != hipSuccess ||
+      vector(&c->dyp, D.J) != hipSuccess ||
+      vector(&c->dzp, D.K) != hipSuccess ||
+      vector(&c->dxu, D.I) != hipSuccess ||
+      vector(&c->dyv, D.J) != hipSuccess ||
+      vector(&c->dzw, D.K) != hipSuccess) {
     sp_destroy(c);
     return SP_ERR_OOM;
   }
@@ -534,6 +591,16 @@ sp_status sp_set_params(sp_ctx* c, const sp_params* p) {
     return fail(c, SP_ERR_INVALID_ARG, "sp_set_params cannot change the grid size");
   c->prm = *p;
   c->have_forward = false;
+  return SP_OK;
+}
+
+sp_status sp_set_solver_memory(sp_ctx* c, int64_t bytes) {
+  if (!c) return SP_ERR_INVALID_ARG;
+  if (bytes < 0) return fail(c, SP_ERR_INVALID_ARG, "solver memory must be >= 0");
+  hipSetDevice(c->device);
+  zring_drop(c);
+  c->zlimit = bytes;
+  c->zdue = true;
   return SP_OK;
 }
 

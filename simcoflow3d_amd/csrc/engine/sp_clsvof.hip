@@ -163,7 +163,7 @@ sp_status interpolate_lvs(sp_ctx* c, const sp_solid_body& B, const sp_lvs_grid& 
   std::vector<void*> tmp;
   auto release = [&]() { for (void* p : tmp) hipFree(p); tmp.clear(); };
   auto stage = [&](const void* src, size_t bytes, bool upload, void** dst) -> sp_status {
-    hipError_t e = hipMalloc(dst, bytes);
+    hipError_t e = dev_malloc(c, dst, bytes);
     if (e != hipSuccess) return hip_check(c, e, "hipMalloc(interpolate_lvs staging)");
     tmp.push_back(*dst);
     if (upload) e = hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, c->stream);

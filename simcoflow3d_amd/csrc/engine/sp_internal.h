@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -15,6 +16,8 @@ constexpr int kMaxLevels = 24;
 constexpr int kTailLdsBytes = 144 * 1024;  // LDS of the V-cycle's tail workgroup
 constexpr int kRedBlockThreads = 256;
 constexpr int kZRing = 16;  // preconditioned residuals kept before x is formed from them
+constexpr int64_t kZRingBytes = (int64_t)8 << 30;  // most memory for them, and
+constexpr int kZRingShare = 16;                    // one part in so many of what is free
 
 // Scalars of the outer CG, resident in device memory so no host round trip
 // is needed between the kernels of one iteration.
@@ -146,9 +149,13 @@ struct sp_ctx {
   bool xd_active = false;
   float* r32 = nullptr;
   // preconditioned residuals of the last CG steps (FP32 with an FP32 V-cycle),
-  // zdepth of them; zring[0] always exists
+  // zdepth of them; zring[0] always exists, the others lie in zslab
   void* zring[sp::kZRing] = {};
   int zdepth = 0;
+  void* zslab = nullptr;
+  int64_t zlimit = sp::kZRingBytes;  // most bytes of zslab
+  bool zdue = false;                 // zslab is to be taken with the next projection
+  std::mutex zmutex;  // held by a solve; whoever gives zslab back waits for it
 
   // multigrid hierarchies (only one is populated, by precision)
   int levels = 0;
@@ -217,6 +224,11 @@ struct RedSite;
 // ---- host helpers (sp_api.hip) ----
 sp_status fail(sp_ctx* c, sp_status s, const std::string& msg);
 sp_status hip_check(sp_ctx* c, hipError_t e, const char* what);
+// Device memory for the context.  The z rings are memory that a solve can do
+// without: when the device has no room, all that the process holds on it are
+// given back (after the solves that use them) and the allocation is tried
+// again.
+hipError_t dev_malloc(sp_ctx* c, void** p, size_t bytes);
 void timer_begin(sp_ctx* c, const char* name, double bytes, int* slot);
 void timer_end(sp_ctx* c, int slot);
 

@@ -1334,6 +1334,8 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
     hipLaunchKernelGGL(kern, dim3(1), dim3(kFinThreads), 0, c->stream, A, nb);
     timer_end(c, slot);
   };
+  // the ring stays this context's until the solve is over
+  std::lock_guard<std::mutex> ring(c->zmutex);
   auto enqueue_residual = [&](int from_zero) {
     A.site = red_site(c, kSiteResidual);
     timer_begin(c, "cg_residual", NB * ((from_zero ? 8 + 1 : 8 * 5 + eb + 1) + 8 + (A.r32 ? 4 : 0)),

@@ -215,7 +215,7 @@ sp_status write_vtr(sp_ctx* c, const char* dir, const char* prefix, int64_t itt,
       const double* src = q < 9 ? cell[q] : coord[q - 9];
       const int64_t n = q < 9 ? (halo[q] ? Nh : N) : (q == 9 ? I : (q == 10 ? J : K));
       void* d = nullptr;
-      hipError_t e = hipMalloc(&d, sizeof(double) * (size_t)n);
+      hipError_t e = dev_malloc(c, &d, sizeof(double) * (size_t)n);
       if (e != hipSuccess) { release(); return hip_check(c, e, "hipMalloc(VTR staging)"); }
       tmp.push_back(d);
       e = hipMemcpyAsync(d, src, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream);
@@ -228,7 +228,7 @@ sp_status write_vtr(sp_ctx* c, const char* dir, const char* prefix, int64_t itt,
   Writer w;
   w.c = c;
   w.cap = text_bytes(kChunk);
-  hipError_t e = hipMalloc(&w.dtext, (size_t)w.cap);
+  hipError_t e = dev_malloc(c, reinterpret_cast<void**>(&w.dtext), (size_t)w.cap);
   if (e == hipSuccess) e = hipHostMalloc(&w.htext, (size_t)w.cap, hipHostMallocDefault);
   if (e != hipSuccess) {
     if (w.dtext) hipFree(w.dtext);
@@ -417,7 +417,7 @@ sp_status write_vtk(sp_ctx* c, const char* dir, int64_t itt, const sp_vtk_fields
       const int axis = (q - 8) % 3;
       const int64_t n = q < 8 ? (halo[q] ? Nh : N) : (axis == 0 ? I : (axis == 1 ? J : K));
       void* d = nullptr;
-      hipError_t e = hipMalloc(&d, sizeof(double) * (size_t)n);
+      hipError_t e = dev_malloc(c, &d, sizeof(double) * (size_t)n);
       if (e != hipSuccess) { release(); return hip_check(c, e, "hipMalloc(VTK staging)"); }
       tmp.push_back(d);
       e = hipMemcpyAsync(d, src, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream);
@@ -430,7 +430,7 @@ sp_status write_vtk(sp_ctx* c, const char* dir, int64_t itt, const sp_vtk_fields
   char* dtext = nullptr;
   char* htext = nullptr;
   const size_t cap = (size_t)(4 * kGroups);
-  hipError_t e = hipMalloc(&dtext, cap);
+  hipError_t e = dev_malloc(c, reinterpret_cast<void**>(&dtext), cap);
   if (e == hipSuccess) e = hipHostMalloc(&htext, cap, hipHostMallocDefault);
   if (e != hipSuccess) {
     if (dtext) hipFree(dtext);

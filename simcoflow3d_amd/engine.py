@@ -40,7 +40,7 @@ EXPORTED_SYMBOLS = (
     "sp_write_vtk", "sp_grid_preprocess", "sp_grid_preprocess_dev", "sp_define_momentum_exchange_cell",
     "sp_number_external_cell", "sp_new_cell_face", "sp_compute_uvw_liquid_field",
     "sp_number_external_cell_noalloc", "sp_predict_uvw", "sp_interpolate_lvs",
-    "sp_clsvof_scheme",
+    "sp_clsvof_scheme", "sp_set_solver_memory",
 )
 
 # members of sp_liquid_field, in order
@@ -266,6 +266,8 @@ def load():
     L.sp_destroy.restype = ctypes.c_int
     L.sp_set_params.argtypes = [V, P(SpParams)]
     L.sp_set_params.restype = ctypes.c_int
+    L.sp_set_solver_memory.argtypes = [V, ctypes.c_int64]
+    L.sp_set_solver_memory.restype = ctypes.c_int
     L.sp_set_grid.argtypes = [V] + [F64P] * 6
     L.sp_set_grid.restype = ctypes.c_int
     L.sp_set_grid_1d.argtypes = [V] + [F64P] * 6
@@ -380,6 +382,11 @@ class Projector:
         for k, v in kw.items():
             setattr(self.params, k, v)
         self._check(self.lib.sp_set_params(self.h, ctypes.byref(self.params)), "sp_set_params")
+
+    def set_solver_memory(self, nbytes):
+        """Most device memory the solver keeps beyond what it cannot do without
+        (default 8 GiB, 0: none)."""
+        self._check(self.lib.sp_set_solver_memory(self.h, nbytes), "sp_set_solver_memory")
 
     def set_grid_1d(self, dxp, dyp, dzp, dxu, dyv, dzw):
         arrs = [np.ascontiguousarray(a, dtype=np.float64) for a in (dxp, dyp, dzp, dxu, dyv, dzw)]
