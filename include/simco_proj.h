@@ -219,8 +219,8 @@ sp_status sp_set_params(sp_ctx* ctx, const sp_params* params);
  * 8 GiB; 0: none, every step then updates the pressure by itself (slower).
  * At most a sixteenth of the device's free memory is taken, with the first
  * projection; it is given back when an allocation of any context of the
- * process finds no room on the device, and with sp_destroy.  Takes effect with
- * the next projection. */
+ * process finds no room on the device, and with sp_destroy.  Results do not
+ * depend on it.  Takes effect with the next projection. */
 sp_status sp_set_solver_memory(sp_ctx* ctx, int64_t bytes);
 
 /* Grid (Mesh.f90:14-18): PGrid%dx,dy,dz and the staggered centre distances

@@ -155,7 +155,7 @@ hipError_t dev_malloc(sp_ctx* c, void** p, size_t bytes) {
 // The buffers of the z ring behind the first: as many as zlimit and a part of
 // the device's free memory hold, in one allocation, none when it is refused.
 // A ring that was given back is not taken again before the buffers are made
-// anew.
+// anew.  The depth does not show in the results (k_cg_xflush).
 static void zring_take(sp_ctx* c) {
   c->zdue = false;
   c->zdepth = 1;

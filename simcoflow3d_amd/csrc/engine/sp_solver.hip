@@ -839,14 +839,15 @@ __global__ void __launch_bounds__(256) k_cg_update(CgArgs A) {
   block_partials<kTileThreads, 2, 1u>(A.site, v);
 }
 
-// x from the kept z of the steps since the last such pass:
-//   x_new = x + sum_j gamma_j (z_j - m_j) + gamma_b p,
-//   gamma_last = alpha_last,  gamma_j = alpha_j + beta_{j+1} gamma_{j+1},
-//   gamma_b = beta_0 gamma_0,
-// on active cells (0 elsewhere), from x = 0 when `assign`.  m is taken off
-// each z before the sum: in a two-phase system the stiff phase's z sits close
-// to m, and its differences matter.  With `keep_p` (a full history in the
-// middle of a solve) p becomes the current direction, from the same z.
+// x from the kept z of the steps since the last such pass, one step after the
+// other as a CG that carries p and x would form them:
+//   p = (z_j - m_j) + beta_j p,   x += alpha_j p
+// on active cells (0 elsewhere), from x = 0 when `assign`.  Fused
+// multiply-adds in a fixed order, so x is the same to the last bit whatever
+// number of z one pass covers: it does not depend on the memory there was for
+// them.  m is taken off each z before the sum: in a two-phase system the stiff
+// phase's z sits close to m, and its differences matter.  With `keep_p` (a
+// full history in the middle of a solve) p is kept for the next pass.
 // z, x and the mask are read and x is written once: 15 steps of an FP32
 // V-cycle at 256^3 move 69 B a cell here, where carrying x and p through the
 // iterations moved 32 B a cell in each of them.
@@ -859,57 +860,35 @@ template <typename Z>
 __global__ void __launch_bounds__(256) k_cg_xflush(CgArgs A, ZHist<Z> H, int64_t N, int assign,
                                                    int keep_p) {
   const Scalars* S = A.S;
-  __shared__ double gam[kZRing], pi[kZRing], sm[kZRing], base[2];
   const int nh = S->nhist;
-  if (threadIdx.x == 0) {
-    double g = 0.0, w = 1.0;
-    for (int j = nh - 1; j >= 0; --j) {
-      g = S->hist_alpha[j] + g;
-      gam[j] = g;
-      pi[j] = w;
-      sm[j] = S->hist_m[j];
-      g *= S->hist_beta[j];
-      w *= S->hist_beta[j];
-    }
-    base[0] = g;
-    base[1] = w;
-  }
-  __syncthreads();
   const int64_t n0 = (int64_t)blockIdx.x * (256 * kFlushCells) + threadIdx.x;
-  double xa[kFlushCells], pa[kFlushCells];
+  double x[kFlushCells], p[kFlushCells];
   bool act[kFlushCells];
-  const double gb = nh > 0 ? base[0] : 0.0, pb = base[1];
+  // beta of a solve's first step is 0, and p is not written before
+  const bool old = nh > 0 && S->hist_beta[0] != 0.0;
 #pragma unroll
   for (int u = 0; u < kFlushCells; ++u) {
     const int64_t n = min(n0 + 256 * u, N - 1);
     act[u] = A.active[n] != 0;
-    xa[u] = assign ? 0.0 : A.x[n];
-    pa[u] = 0.0;
-    // beta of a solve's first step is 0, and p is not written before
-    if (gb != 0.0 || (keep_p && pb != 0.0)) {
-      const double p = A.p[n];
-      xa[u] += gb * p;
-      pa[u] = pb * p;
-    }
+    x[u] = assign ? 0.0 : A.x[n];
+    p[u] = old ? A.p[n] : 0.0;
   }
 #pragma unroll 4
   for (int j = 0; j < nh; ++j) {
-    const double g = gam[j], w = pi[j], m = sm[j];
+    const double alpha = S->hist_alpha[j], beta = S->hist_beta[j], m = S->hist_m[j];
     const Z* z = H.z[j];
 #pragma unroll
     for (int u = 0; u < kFlushCells; ++u) {
-      const int64_t n = min(n0 + 256 * u, N - 1);
-      const double zv = (double)z[n] - m;
-      xa[u] += g * zv;
-      pa[u] += w * zv;
+      p[u] = fma(beta, p[u], (double)z[min(n0 + 256 * u, N - 1)] - m);
+      x[u] = fma(alpha, p[u], x[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < kFlushCells; ++u) {
     const int64_t n = n0 + 256 * u;
     if (n >= N) break;
-    A.x[n] = act[u] ? xa[u] : 0.0;
-    if (keep_p) A.p[n] = act[u] ? pa[u] : 0.0;
+    A.x[n] = act[u] ? x[u] : 0.0;
+    if (keep_p && nh > 0) A.p[n] = act[u] ? p[u] : 0.0;
   }
 }
 __global__ void k_cg_hist_reset(Scalars* S) { S->nhist = 0; }

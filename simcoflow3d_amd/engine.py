@@ -385,7 +385,7 @@ class Projector:
 
     def set_solver_memory(self, nbytes):
         """Most device memory the solver keeps beyond what it cannot do without
-        (default 8 GiB, 0: none)."""
+        (default 8 GiB, 0: none); results do not depend on it."""
         self._check(self.lib.sp_set_solver_memory(self.h, nbytes), "sp_set_solver_memory")
 
     def set_grid_1d(self, dxp, dyp, dzp, dxu, dyv, dzw):

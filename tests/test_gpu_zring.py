@@ -2,6 +2,7 @@
 a solve stopped after m steps must return the x that its recursive residual
 belongs to, on both sides of every ring boundary."""
 
+import numpy as np
 import pytest
 
 from tests import helpers as H
@@ -25,3 +26,34 @@ def test_iterate_belongs_to_its_residual(gpu_available, kw, steps):
     assert st.iterations == steps
     assert st.residual_div < st.initial_div
     assert abs(st.final_div - st.residual_div) <= 1e-12 * st.initial_div
+
+
+@pytest.mark.parametrize("kw", [dict(precision=1, mg_levels=2), dict(precision=0, mg_levels=2),
+                                dict(precision=0, precond=1),
+                                dict(precision=1, mg_levels=2, flags=2)])
+@pytest.mark.parametrize("steps", [7, 400])
+def test_result_does_not_depend_on_the_depth(gpu_available, kw, steps):
+    """Rings of 1, 2, 4, 8 and 16 (sp_set_solver_memory): the same iterations
+    and the same bytes, for a solve cut short and for one that converges over
+    several rings; with an outlet, whose refinement solves again, too."""
+    size = (33, 20, 26)
+    z = size[0] * size[1] * size[2] * (4 if kw["precision"] and not kw.get("precond") else 8) + 512
+    for cfg, bc in ((2, None), (4, 1)):
+        c = H.case(cfg, size=size)
+        flag, val = list(c.bc_flag), None
+        if bc is not None:
+            flag[bc], val = 0, [None] * 6
+            val[bc] = np.zeros((c.J, c.K), order="F")
+        first = None
+        for depth in (16, 1, 2, 4, 8):
+            print(f"[zring] {kw} steps={steps} cfg={cfg} depth={depth}", flush=True)
+            P = H.projector(c, max_iter=steps, **kw)
+            P.set_solver_memory((depth - 1) * z)
+            out, st = P.project(H.fields(c), flag, c.dt, bc_val=val)
+            P.close()
+            assert steps == 7 or st.iterations > 16
+            if first is None:
+                first = out, st.iterations
+            assert st.iterations == first[1]
+            for n in ("p", "u", "v", "w"):
+                assert np.array_equal(out[n], first[0][n]), (depth, n)
