@@ -191,6 +191,14 @@ __global__ void __launch_bounds__(256) k_prolong(LevelView<T> F, LevelView<T> C,
 // read from global memory two levels (8^3 and 4^3) took 22 us a cycle, and a
 // 16^3 level was better off in legs of 9 us (FP32) each; here the three levels
 // take 21 us in FP32 and 29 in FP64 (event times, 5 us of them the launch).
+//
+// BIG = 4: a coarsest level alone with four pairs per thread, for one that two
+// do not hold (a hierarchy cut short, a grid too thin to coarsen).  In FP32
+// the couplings of four still fit the registers (FP64 spills with two).  It
+// beats one launch per half-sweep over the whole chip, and keeps the mean out
+// of a singular system's coarse solve, up to the last size it holds (whole
+// solves: 40 x 40 x 3 7.25 -> 5.29 ms, 50 x 50 x 2 6.81 -> 5.05, one level of
+// 18^3 3.34 -> 2.96, of 20^3 3.65 -> 3.41, of 24 x 24 x 14 3.82 -> 3.55).
 constexpr int kTailThreads = 1024, kTailLevels = 8;
 
 template <typename T>
@@ -206,6 +214,8 @@ struct TailArgs {
   T* x;
 };
 
+template <typename T>
+int64_t tail_pairs(const Level<T>& L) { return (int64_t)((L.nx + 1) / 2) * L.ny * L.nz; }
 // Threads that a level's pairs take, in whole waves.
 inline int tail_threads(int nx, int ny, int nz) { return ((nx + 1) / 2 * ny * nz + 63) / 64 * 64; }
 
@@ -299,23 +309,24 @@ __device__ inline void tail_load(TailPair<T, HAS_E>& P, const TailArgs<T>& A, in
   }
 }
 
-// The workgroup's state.  TOP: the first level (two pairs of every thread),
+// The workgroup's state.  TOP: the first level (BIG pairs of every thread),
 // otherwise level l (one pair of the threads with mine == l); the two are told
 // apart at compile time so that the pairs stay in registers.
-template <typename T, bool HAS_E>
+template <typename T, bool HAS_E, int BIG>
 struct Tail {
   using Pair = TailPair<T, HAS_E>;
   const TailArgs<T>& A;
   T* xs;
   double (*red)[kTailThreads / 64];
-  Pair big[2], small;
+  Pair big[BIG], small;
   int t, mine;
 
   template <bool TOP, typename F>
   __device__ __forceinline__ void own(int l, F f) {
     if constexpr (TOP) {
-      if (big[0].any) f(big[0]);
-      if (big[1].any) f(big[1]);
+#pragma unroll
+      for (int p = 0; p < BIG; ++p)
+        if (big[p].any) f(big[p]);
     } else if (mine == l && small.any) {
       f(small);
     }
@@ -433,25 +444,28 @@ struct Tail {
   }
 };
 
-template <typename T, bool HAS_E>
+template <typename T, bool HAS_E, int BIG>
 __global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A, const Scalars* S) {
   if (S->done) return;
+  constexpr bool kAlone = BIG > 2;
   __shared__ double lds_raw[kTailLdsBytes / sizeof(double)];
   __shared__ double red[2][kTailThreads / 64];
-  Tail<T, HAS_E> W{A, reinterpret_cast<T*>(lds_raw), red, {}, {}, (int)threadIdx.x, 0};
-  tail_load(W.big[0], A, 0, W.t);
-  tail_load(W.big[1], A, 0, W.t + kTailThreads);
-  for (int l = 1; l < A.n; ++l)
-    if (W.t >= A.first[l]) W.mine = l;
-  W.small.any = false;
-  if (W.mine) tail_load(W.small, A, W.mine, W.t - A.first[W.mine]);
+  Tail<T, HAS_E, BIG> W{A, reinterpret_cast<T*>(lds_raw), red, {}, {}, (int)threadIdx.x, 0};
+#pragma unroll
+  for (int p = 0; p < BIG; ++p) tail_load(W.big[p], A, 0, W.t + p * kTailThreads);
+  if constexpr (!kAlone) {
+    for (int l = 1; l < A.n; ++l)
+      if (W.t >= A.first[l]) W.mine = l;
+    W.small.any = false;
+    if (W.mine) tail_load(W.small, A, W.mine, W.t - A.first[W.mine]);
+  }
   // the x arrays lie before the residuals
   for (int q = W.t; q < A.ro[0]; q += kTailThreads) W.xs[q] = T(0);
   __syncthreads();
-  const int last = A.n - 1;
+  const int last = kAlone ? 0 : A.n - 1;
   if (last == 0) {
     W.template coarsest<true>(0);
-  } else {
+  } else if constexpr (!kAlone) {
     W.template down<true>(0);
     for (int l = 1; l < last; ++l) W.template down<false>(l);
     W.template coarsest<false>(last);
@@ -459,7 +473,7 @@ __global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A, const Scal
     W.template up<true>(0);
   }
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
+  for (int p = 0; p < BIG; ++p)
 #pragma unroll
     for (int q = 0; q < 2; ++q)
       if (W.big[p].exists(q)) A.x[W.big[p].cell(q)] = W.xs[W.big[p].at[q]];
@@ -1167,12 +1181,15 @@ void vcycle(sp_ctx* c, Level<T>* lv) {
       off += (int)lv[Lt + q].n;
     }
     timer_begin(c, "mg_tail", 0, &slot);
-    if (lv[Lt].e)
-      hipLaunchKernelGGL((k_tail<T, true>), dim3(1), dim3(kTailThreads), 0, c->stream, A,
-                         (const Scalars*)c->S);
-    else
-      hipLaunchKernelGGL((k_tail<T, false>), dim3(1), dim3(kTailThreads), 0, c->stream, A,
-                         (const Scalars*)c->S);
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(1), dim3(kTailThreads), 0, c->stream, A, (const Scalars*)c->S);
+    };
+    bool wide = false;
+    if constexpr (sizeof(T) == 4) {
+      wide = tail_pairs(lv[Lt]) > 2 * kTailThreads;
+      if (wide) lv[Lt].e ? launch(k_tail<T, true, 4>) : launch(k_tail<T, false, 4>);
+    }
+    if (!wide) lv[Lt].e ? launch(k_tail<T, true, 2>) : launch(k_tail<T, false, 2>);
     timer_end(c, slot);
   }
   for (int l = Lp - 1; l >= 0; --l) {
@@ -1220,8 +1237,8 @@ sp_status setup_levels(sp_ctx* c, Level<T>* lv) {
 }  // namespace
 
 // The first level of the tail kernel (c->tail_level): the levels from it on
-// fit its threads (two pairs each on the first level, one on the others) and
-// LDS.  c->levels when not even the coarsest level does (a hierarchy cut short
+// fit its threads (two pairs each on the first level, one on the others; four
+// on a coarsest level alone in FP32) and LDS.  c->levels when not even the coarsest level does (a hierarchy cut short
 // by mg_levels, or a large grid that cannot coarsen): the V-cycle then smooths
 // the coarsest level in global memory.
 template <typename T>
@@ -1234,8 +1251,9 @@ static int first_tail_level(const Level<T>* lv, int levels) {
              ((int64_t)(lv[q].nx + 2) * (lv[q].ny + 2) * (lv[q].nz + 2) + lv[q].n);
       if (q > l && lv[q].n <= 4 * kTailThreads) threads += tail_threads(lv[q].nx, lv[q].ny, lv[q].nz);
     }
-    const int64_t pairs = (int64_t)((lv[l].nx + 1) / 2) * lv[l].ny * lv[l].nz;
-    if (pairs > 2 * kTailThreads || threads > kTailThreads || lds > kTailLdsBytes) break;
+    const int big = sizeof(T) == 4 && l == levels - 1 ? 4 : 2;
+    if (tail_pairs(lv[l]) > big * kTailThreads || threads > kTailThreads || lds > kTailLdsBytes)
+      break;
     best = l;
   }
   return best;
