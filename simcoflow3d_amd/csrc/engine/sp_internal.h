@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "simco_proj.h"
+#include "sp_legs.h"
 
 namespace sp {
 
@@ -90,6 +91,8 @@ struct Level {
   T* xs;       // pre-smoothed x (input of the fused post-smoother); the
                // Chebyshev smoother's second iterate buffer
   T* cd;       // the Chebyshev smoother's direction
+  LegGrid leg;  // launch of the smoother legs, set with the couplings
+  bool four;    // FP32: they take four cells per thread
 };
 
 struct Dims {

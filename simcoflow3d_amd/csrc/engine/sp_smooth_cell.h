@@ -6,13 +6,8 @@
 // computes both colours' half-sweeps and keeps those of its own.  That wastes
 // half of the arithmetic, but a step is a shorter chain and a thread holds
 // one window of each array.  It is the better one
-//   * on levels of few columns, which give too few large tiles to put one on
-//     every CU and whose march is a few steps long and bound by the latency of
-//     a step (per leg, pre and post, event times, four cells per thread
-//     against this: 80^3 19.5 and 19.1 against 16.2 and 17.5 us, 96^3 21.4 and
-//     21.7 against 17.6 and 18.9, 112^3 23.6 and 24.4 against 21.7 and 22.9,
-//     97 x 130 x 75 22.1 and 22.4 against 22.4 and 25.1, 128^3 24.3 and 26.0
-//     against 23.8 and 24.9, 256^3 105 and 116 against 117 and 140);
+//   * where the large tiles do not shorten the march enough (small levels,
+//     thin ones): a step is bound by its latency there (four_cell_leg);
 //   * with a diagonal-only term, whose windows do not fit the registers two or
 //     four times (160 x 96 x 96 with an outlet, whole solve: 2.88 ms against
 //     3.16 with a pair and 3.96 with four, which spills).
@@ -25,11 +20,6 @@
 #include "sp_smooth_fused.h"
 
 namespace sp {
-
-constexpr int64_t kCellColumns = 112 * 112;  // most columns of an FP32 level for it
-
-constexpr int kFEX = 40;  // extended tile width (threads along i)
-constexpr int kFEY = 24;  // extended tile height (threads along j)
 
 // Coarse levels too small in (i, j) to fill the chip with extended 40 x 24
 // tiles march with 16 x 16 (an 8 x 8 interior at NU = 2): four waves per

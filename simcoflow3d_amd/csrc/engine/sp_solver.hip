@@ -994,23 +994,45 @@ void launch_cheb(sp_ctx* c, const Level<T>& L, int m, bool from_zero, bool fine)
     hipMemcpyAsync(L.x, in, sizeof(T) * (size_t)L.n, hipMemcpyDeviceToDevice, c->stream);
 }
 
-// Grid of a smoother leg, and its k chunk: even (coarse cells never straddle
-// chunks).  A workgroup marches kchunk + 2H planes one after the other, so pick
-// the chunk that minimises rounds-of-workgroups x planes marched.
+// Launch of a level's legs with tiles of Sh, per_cu workgroups on a CU at once.
 template <typename Sh, typename T>
-dim3 leg_grid(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, int per_cu) {
-  const int gx = (L.nx + Sh::TX - 1) / Sh::TX, gy = (L.ny + Sh::TY - 1) / Sh::TY;
-  const int64_t tiles = (int64_t)gx * gy, slots = (int64_t)std::max(1, c->num_cu) * per_cu;
-  const int kmax = (L.nz + 1) & ~1;
-  int64_t best_cost = -1;
-  for (int kc = 2; kc <= kmax; kc += 2) {
-    const int64_t blocks = tiles * ((L.nz + kc - 1) / kc);
-    const int64_t cost = ((blocks + slots - 1) / slots) * (kc + 2 * Sh::H);
-    if (best_cost < 0 || cost < best_cost) { best_cost = cost; A.kchunk = kc; }
-  }
-  const dim3 grd(gx, gy, (L.nz + A.kchunk - 1) / A.kchunk);
-  if (A.dots) c->dots_nb = grd.x * grd.y * grd.z;
-  return grd;
+LegGrid leg_of(const sp_ctx* c, const Level<T>& L, int per_cu) {
+  return leg_grid(L.nx, L.ny, L.nz, Sh::TX, Sh::TY, Sh::H,
+                  (int64_t)std::max(1, c->num_cu) * per_cu);
+}
+
+// Small tiles for the levels below the finest of at most 32 x 32 columns:
+// these have two 32 x 16 tiles, whose 10-step marches (2 planes + the 8-plane
+// pipeline) run on 32 CUs.  Small tiles put a workgroup on every CU (32^3:
+// 10.5 -> 7.8 us per leg); at 64 x 64 they measured slower than the large ones
+// (13.0 against 11.7 us).
+template <typename T>
+bool small_legs(const Level<T>& L, bool fine) {
+  return !fine && (int64_t)L.nx * L.ny <= 32 * 32;
+}
+
+// FP32: four cells per thread or one (four_cell_leg); one with a diagonal-only
+// term.
+template <int NU>
+void plan_legs(const sp_ctx* c, Level<float>& L, bool fine) {
+  using Four = FusedTile<float, false>;
+  static_assert(Four::Q == 2 && 4 * Four::EP == kQEX && Four::EY == kQEY && Four::kPerCu == 1,
+                "four_cell_leg weighs these tiles");
+  L.four = !small_legs(L, fine) && !L.e &&
+           four_cell_leg(L.nx, L.ny, L.nz, NU, std::max(1, c->num_cu));
+  if (small_legs(L, fine)) L.leg = leg_of<CellShape<NU, kFEXs, kFEYs>>(c, L, 4);
+  else if (L.four) L.leg = leg_of<FusedShape<NU, Four::Q, Four::EP, Four::EY>>(c, L, 1);
+  else L.leg = leg_of<CellShape<NU, kFEX, kFEY>>(c, L, 1);
+}
+template <int NU, bool SMALL>
+void plan_legs64(const sp_ctx* c, Level<double>& L) {
+  using Tile = FusedTile<double, SMALL>;
+  L.leg = leg_of<FusedShape<NU, Tile::Q, Tile::EP, Tile::EY>>(c, L, Tile::kPerCu);
+}
+template <int NU>
+void plan_legs(const sp_ctx* c, Level<double>& L, bool) {
+  if ((int64_t)L.nx * L.ny <= kSmallColumns) plan_legs64<NU, true>(c, L);
+  else plan_legs64<NU, false>(c, L);
 }
 
 // One smoother leg.  KERNEL(MODE, FINE): the kernel of a form.
@@ -1025,7 +1047,7 @@ template <typename T, int NU, bool HAS_E, bool SMALL>
 void launch_march(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode) {
   using Tile = FusedTile<T, SMALL>;
   constexpr int Q = Tile::Q, EP = Tile::EP, EY = Tile::EY;
-  const dim3 grd = leg_grid<FusedShape<NU, Q, EP, EY>>(c, L, A, Tile::kPerCu), blk(EP * EY, 1, 1);
+  const dim3 grd(L.leg.gx, L.leg.gy, L.leg.gz), blk(EP * EY, 1, 1);
   const Scalars* S = c->S;
 #define SP_K(MODE, FINE) k_smooth_fused<T, NU, Q, MODE, FINE, HAS_E, EP, EY>
   SP_LEG(SP_K);
@@ -1033,8 +1055,8 @@ void launch_march(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int 
 }
 
 template <typename T, int NU, bool HAS_E, int EX, int EY>
-void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode, int per_cu) {
-  const dim3 grd = leg_grid<CellShape<NU, EX, EY>>(c, L, A, per_cu), blk(EX, EY, 1);
+void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode) {
+  const dim3 grd(L.leg.gx, L.leg.gy, L.leg.gz), blk(EX, EY, 1);
   const Scalars* S = c->S;
 #define SP_K(MODE, FINE) k_smooth_cell<T, NU, MODE, FINE, HAS_E, EX, EY>
   SP_LEG(SP_K);
@@ -1042,25 +1064,16 @@ void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int m
 }
 #undef SP_LEG
 
-// FP32: four cells per thread on levels without a diagonal-only term and of
-// more than kCellColumns columns, else one cell per thread.
 template <int NU>
 void launch_leg(sp_ctx* c, const Level<float>& L, FusedArgs<float>& A, bool fine, int mode) {
-  const int64_t cols = (int64_t)L.nx * L.ny;
-  if (!A.e && cols > kCellColumns) {
+  if (small_legs(L, fine)) {
+    if (A.e) launch_cell<float, NU, true, kFEXs, kFEYs>(c, L, A, fine, mode);
+    else launch_cell<float, NU, false, kFEXs, kFEYs>(c, L, A, fine, mode);
+  } else if (L.four) {
     launch_march<float, NU, false, false>(c, L, A, fine, mode);
-    return;
-  }
-  // a level of at most 32 x 32 columns has two 32 x 16 tiles: its 10-step
-  // marches (2 planes + the 8-plane pipeline) run on 32 CUs.  Small tiles put
-  // a workgroup on every CU (32^3: 10.5 -> 7.8 us per leg); at 64 x 64 they
-  // measured slower than the large ones (13.0 against 11.7 us)
-  if (!fine && cols <= 32 * 32) {
-    if (A.e) launch_cell<float, NU, true, kFEXs, kFEYs>(c, L, A, fine, mode, 4);
-    else launch_cell<float, NU, false, kFEXs, kFEYs>(c, L, A, fine, mode, 4);
   } else {
-    if (A.e) launch_cell<float, NU, true, kFEX, kFEY>(c, L, A, fine, mode, 1);
-    else launch_cell<float, NU, false, kFEX, kFEY>(c, L, A, fine, mode, 1);
+    if (A.e) launch_cell<float, NU, true, kFEX, kFEY>(c, L, A, fine, mode);
+    else launch_cell<float, NU, false, kFEX, kFEY>(c, L, A, fine, mode);
   }
 }
 template <int NU>
@@ -1083,12 +1096,14 @@ void launch_fused(sp_ctx* c, Level<T>* lv, int l, int mode) {
   A.cx = L.cx; A.cy = L.cy; A.cz = L.cz; A.e = L.e;
   A.b = L.b;
   A.cnx = C.nx; A.cny = C.ny;
+  A.kchunk = L.leg.kchunk;
   A.omega = (T)(l == 0 ? c->prm.mg_omega : c->prm.mg_omega_coarse);
   if (mode == 0) { A.xout = L.xs; A.bc = C.b; }
   else { A.xin = L.xs; A.xc = C.x; A.xout = L.x; }
   if (mode == 1 && l == 0 && c->fuse_dots) {
     A.dots = 1;
     A.dsite = red_site(c, kSiteDots);
+    c->dots_nb = (uint32_t)L.leg.gx * L.leg.gy * L.leg.gz;
   }
   const bool fine = l == 0;
   int slot;
@@ -1230,6 +1245,12 @@ sp_status setup_levels(sp_ctx* c, Level<T>* lv) {
     hipLaunchKernelGGL(k_coarsen<T>, flat_grid(C.nx, C.ny, C.nz), blk, 0, c->stream,
                        view_of(lv[l - 1]), view_of(C), C.cx, C.cy, C.cz, C.e,
                        (T)c->prm.mg_coarse_scale);
+  }
+  if (fused_vcycle(c)) {
+    for (int l = 0; l < L; ++l) {
+      if (c->prm.mg_pre == 2) plan_legs<2>(c, lv[l], l == 0);
+      else plan_legs<1>(c, lv[l], l == 0);
+    }
   }
   return SP_OK;
 }
