@@ -8,6 +8,7 @@ import subprocess
 import pytest
 
 from simcoflow3d_amd._paths import PKG_DIR
+from tests import test_gpu_smoother_tiles as tiles
 
 PROGRAM = r"""
 #include <cstdio>
@@ -51,6 +52,16 @@ def ask(tmp_path_factory):
 def test_measured_sizes_take_the_faster_form(ask):
     assert [c for c, r in zip(FOUR, ask(FOUR)) if r[0] != 4] == []
     assert [c for c, r in zip(ONE, ask(ONE)) if r[0] != 1] == []
+
+
+def test_sizes_of_the_tile_tests(ask):
+    """The GPU tests of the legs reach the form that they are meant for."""
+    four = [(s, w) for s in tiles.FOUR for w in (1, 2)]
+    four += [(s, 1) for s in tiles.FOUR_1] + [(s, 2) for s in tiles.FOUR_2]
+    assert [c for c, r in zip(four, ask(four)) if r[0] != 4] == []
+    assert {s[0] % 4 for s, w in four if w == 2} == {s[0] % 4 for s, w in four if w == 1} == {0, 1, 2, 3}
+    one = [(s, w) for s in tiles.SIZES for w in (1, 2)]
+    assert [c for c, r in zip(one, ask(one)) if r[0] != 1] == []
 
 
 def test_chunks_cover_the_planes(ask):
