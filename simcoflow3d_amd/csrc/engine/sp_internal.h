@@ -33,7 +33,7 @@ struct Scalars {
   double dsum;      // sum of the diagonal over active cells
   double zshift;    // diagonal-weighted mean of z removed in singular systems
   double src_max;   // max |pbar_i| / V_i of the adjoint source
-  double rsum, qsum;  // sums of r and q over the cells (for the z shift)
+  double rsum;      // sum of r over the cells (for the z shift)
   double npart[8];  // scratch results of small reductions
   // alpha, beta and the shift of z of the CG steps whose z are kept
   double hist_alpha[kZRing], hist_beta[kZRing], hist_m[kZRing];

@@ -398,11 +398,10 @@ __device__ inline void fused_step(FusedState<T, NU, Q>& F, const PlaneLoad<T, Q>
   }
 }
 
-// Planes of loads in flight: what the registers hold (FP64, or four cells per
-// thread, leave room for fewer; 2, 3 and 6 measured the same where they fit).
-template <typename T, int NU, int Q>
+// Planes of loads in flight: what the registers hold.
+template <typename T>
 constexpr int fused_pipe() {
-  return sizeof(T) == 8 ? 1 : (Q == 1 && NU == 2 ? 3 : 2);
+  return sizeof(T) == 8 ? 1 : 2;
 }
 
 // Steps t + U, t + U + 1, ..., t + W - 1 of the march, each followed by the
@@ -496,7 +495,7 @@ __global__ void __launch_bounds__(EP * EY) k_smooth_fused(FusedArgs<T> A, const 
   // buffer u % P holds the planes of steps t0 + u (mod P)
   const int t0 = k0 - H, t1 = k1 + H;  // steps [t0, t1); t0 even
   constexpr bool DOTS = FINE && MODE == 1;
-  constexpr int P = fused_pipe<T, NU, Q>();
+  constexpr int P = fused_pipe<T>();
   PlaneLoad<T, Q> LB[P];
 #pragma unroll
   for (int u = 0; u < P; ++u) load_plane<T, Q, MODE, HAS_E>(LB[u], A, C, t0 + u);

@@ -657,7 +657,6 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_residual_fin(CgArgs A, uint3
     Scalars* S = A.S;
     S->rmax = out[0];
     S->rsum = out[2];
-    S->qsum = 0.0;
     S->nhist = 0;
     S->nonfinite = S->nonfinite || out[1] > 0.0 || !is_finite(out[0]);
     S->done = (out[0] <= A.tol || S->nonfinite) ? 1 : 0;
@@ -745,7 +744,7 @@ __global__ void __launch_bounds__(kFinThreads) k_cg_dots2_fin(CgArgs A, uint32_t
 
 // The image of the search direction in one pass:
 //   q = A (z - m) + beta q_old
-// with (p, q) = (z - m, q) and sum q for alpha.  A 1 is the diagonal-only
+// with (p, q) = (z - m, q) and (z - m, q_old) for alpha.  A 1 is the diagonal-only
 // term e (the face couplings of a row sum to its diagonal minus e), so the
 // stencil is applied to z, which is complete in memory.  Rows of inactive
 // cells have no couplings and z = 0: q stays 0 there without a mask.  Each
@@ -756,7 +755,7 @@ __global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
   Scalars* S = A.S;
   if (S->done) return;
   const Col3 q = col_of<KC>(A.I, A.J, A.K);
-  double v[3] = {0.0, 0.0, 0.0};  // (z - m, q), sum q, (z - m, q_old)
+  double v[2] = {0.0, 0.0};  // (z - m, q), (z - m, q_old)
   if (q.in) {
     const double beta = S->beta, m = S->zshift;
     const int64_t I = A.I, IJ = (int64_t)A.I * A.J;
@@ -795,29 +794,27 @@ __global__ void __launch_bounds__(256) k_cg_spmv(CgArgs A, const Z* zv) {
       const double qv = (az - m * en) + beta * qo;
       A.q[n] = qv;
       v[0] += (zc - m) * qv;
-      v[1] += qv;
-      v[2] += (zc - m) * qo;
+      v[1] += (zc - m) * qo;
       zm = zc;
       zc = zp;
       czm = cz;
     }
   }
-  block_partials<kTileThreads, 3, 0u>(A.site, v);
+  block_partials<kTileThreads, 2, 0u>(A.site, v);
 }
 
 __global__ void __launch_bounds__(kFinThreads) k_cg_spmv_fin(CgArgs A, uint32_t nb) {
   Scalars* S = A.S;
   if (S->done) return;
-  double t[3];
-  finalize_partials<kFinThreads, 3, 0u>(A.site, nb, t);
+  double t[2];
+  finalize_partials<kFinThreads, 2, 0u>(A.site, nb, t);
   if (flat_tid() == 0) {
     const double beta = S->beta;
     // (p, q) of p = (z - m) + beta p_old, also where beta has left p a little
     // short of A-orthogonal to p_old: alpha then still is the exact minimiser
     // along p (pq holds the last step's value, beta is 0 in the first)
-    const double pq = t[0] + (beta != 0.0 ? beta * (t[2] + beta * S->pq) : 0.0);
+    const double pq = t[0] + (beta != 0.0 ? beta * (t[1] + beta * S->pq) : 0.0);
     S->pq = pq;
-    S->qsum = t[1];
     S->alpha = S->rz / pq;
     S->hist_alpha[A.slot] = S->alpha;
     S->nhist = A.slot + 1;
