@@ -58,6 +58,12 @@ void timer_end(sp_ctx* c, int slot) {
   hipEventRecord(c->ev_pool[slot].second, c->stream);
 }
 
+void timer_bytes(sp_ctx* c, const char* name, double bytes) {
+  if (!c->profiling) return;
+  for (Timer& t : c->timers)
+    if (t.name == name) t.bytes += bytes;
+}
+
 static void timers_collect(sp_ctx* c) {
   if (!c->profiling) return;
   hipStreamSynchronize(c->stream);

@@ -234,6 +234,8 @@ sp_status hip_check(sp_ctx* c, hipError_t e, const char* what);
 hipError_t dev_malloc(sp_ctx* c, void** p, size_t bytes);
 void timer_begin(sp_ctx* c, const char* name, double bytes, int* slot);
 void timer_end(sp_ctx* c, int slot);
+// Bytes that become known after the launches of `name`.
+void timer_bytes(sp_ctx* c, const char* name, double bytes);
 
 // ---- host <-> device copies of pageable arrays (sp_hostio.hip) ----
 sp_status pipe_upload(sp_ctx* c, void* dst, const void* src, size_t bytes);

@@ -1398,12 +1398,12 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
     enqueue_residual(1);
   }
   // x from the kept z (k_cg_xflush); `keep_p`: the solve goes on
-  bool assign = !resume;
+  bool assign = !resume, carried = false;  // carried: p holds the last pass's direction
   auto form_x = [&](bool keep_p) {
     const dim3 grd((unsigned)((D.N + 256 * kFlushCells - 1) / (256 * kFlushCells)));
-    // counts a full history; the last pass of a solve reads what it holds
-    timer_begin(c, "cg_xflush", NB * (zb * c->zdepth + 1 + (assign ? 8 : 16) + (keep_p ? 8 : 0)),
-                &slot);
+    // a full history's z, or what the device then says the last pass read
+    timer_begin(c, "cg_xflush", NB * ((keep_p ? zb * c->zdepth + 8 : 0) + 1 + (assign ? 8 : 16) +
+                                      (carried ? 8 : 0)), &slot);
     if (mixed && mg) {
       ZHist<float> H{};
       for (int j = 0; j < c->zdepth; ++j) H.z[j] = static_cast<const float*>(c->zring[j]);
@@ -1418,6 +1418,7 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
     timer_end(c, slot);
     if (keep_p) hipLaunchKernelGGL(k_cg_hist_reset, dim3(1), dim3(1), 0, c->stream, c->S);
     assign = false;
+    carried = keep_p;
   };
   int restarts = 0;
   const int max_iter = std::max(1, c->prm.max_iter);
@@ -1481,6 +1482,7 @@ sp_status solve(sp_ctx* c, const double* rhs, double tol, sp_stats* st, bool che
     if (e != hipSuccess) { hipEventDestroy(evs[0]); hipEventDestroy(evs[1]); return hip_check(c, e, "solve"); }
     e = hipMemcpy(c->S_host, c->S, sizeof(Scalars), hipMemcpyDeviceToHost);
     if (e != hipSuccess) { hipEventDestroy(evs[0]); hipEventDestroy(evs[1]); return hip_check(c, e, "solve"); }
+    timer_bytes(c, "cg_xflush", NB * zb * c->S_host->nhist);
     const int iters = c->S_host->iter;
     if (c->S_host->nonfinite || !check_true) break;
     // true residual of the final iterate

@@ -57,3 +57,21 @@ def test_result_does_not_depend_on_the_depth(gpu_available, kw, steps):
             assert st.iterations == first[1]
             for n in ("p", "u", "v", "w"):
                 assert np.array_equal(out[n], first[0][n]), (depth, n)
+
+
+@pytest.mark.parametrize("prec", (0, 1))
+@pytest.mark.parametrize("depth", (16, 4))
+def test_bytes_of_the_pass_that_forms_x(gpu_available, prec, depth):
+    """sp_kernel_times counts the z that the pass reads, not the ring."""
+    c = H.case(0, size=(32, 32, 32))
+    n, z = 32 ** 3, 4 if prec else 8
+    print(f"[zring] bytes prec={prec} depth={depth}", flush=True)
+    P = H.projector(c, precision=prec)
+    P.set_solver_memory((depth - 1) * (n * z + 512))
+    P.set_profiling(True)
+    _, st = P.project(H.fields(c), c.bc_flag, c.dt)
+    t = next(k for k in P.kernel_times() if k["name"] == "cg_xflush")
+    P.close()
+    full = t["launches"] - 1  # passes that keep p: it is written, and read by the next
+    assert full == st.iterations // depth  # one more step was under way
+    assert t["bytes"] == n * (z * st.iterations + 9 + full * (9 + 8 + 8 + 8))
