@@ -37,24 +37,12 @@ struct CellShape {
                 "the restriction pairs cells inside the tile interior");
 };
 
-// Element at a 32-bit byte offset (every level array is below 4 GiB), so the
-// loads use a scalar base plus one 32-bit vector offset.
-template <typename T>
-__device__ inline T cell_at(const T* base, uint32_t byte_off) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
-}
-template <typename T>
-__device__ inline void cell_put(T* base, uint32_t byte_off, T v) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte_off) = v;
-}
-
 // Raw loads of one plane.  The loads always target a valid address (the
 // plane index is clamped, neighbours fall back to the cell itself) so their
 // destination registers carry straight into the next pipeline step; validity
 // is applied when the values are consumed.
-template <typename T>
 struct CellLoad {
-  T b, cx, cy, cz, cxm, cym, e, xin, xc;
+  float b, cx, cy, cz, cxm, cym, e, xin, xc;
   bool vt;
 };
 
@@ -70,46 +58,47 @@ struct CellCol {
   uint32_t cplane;       // post: bytes per coarse plane
 };
 
-template <typename T, int MODE, bool HAS_E>
-__device__ inline void cell_load(CellLoad<T>& L, const FusedArgs<T>& A, const CellCol& C, int t) {
+template <int MODE, bool HAS_E>
+__device__ inline void cell_load(CellLoad& L, const FusedArgs<float>& A, const CellCol& C, int t) {
   const int tc = t < 0 ? 0 : (t >= A.nz ? A.nz - 1 : t);
   const uint32_t n = C.col + C.plane * (uint32_t)tc;
   L.vt = C.in_ij && t >= 0 && t < A.nz;
-  L.b = cell_at(A.b, n);
-  L.cx = cell_at(A.cx, n);
-  L.cy = cell_at(A.cy, n);
-  L.cz = cell_at(A.cz, n);
-  L.cxm = cell_at(A.cx, n - C.dxm);
-  L.cym = cell_at(A.cy, n - C.dym);
-  L.e = HAS_E ? cell_at(A.e, n) : T(0);
+  L.b = at_off<float>(A.b, n);
+  L.cx = at_off<float>(A.cx, n);
+  L.cy = at_off<float>(A.cy, n);
+  L.cz = at_off<float>(A.cz, n);
+  L.cxm = at_off<float>(A.cx, n - C.dxm);
+  L.cym = at_off<float>(A.cy, n - C.dym);
+  L.e = HAS_E ? at_off<float>(A.e, n) : 0.f;
   if (MODE == 1) {
-    L.xin = cell_at(A.xin, n);
-    L.xc = cell_at(A.xc, C.ccol + C.cplane * (uint32_t)(tc >> 1));
+    L.xin = at_off<float>(A.xin, n);
+    L.xc = at_off<float>(A.xc, C.ccol + C.cplane * (uint32_t)(tc >> 1));
   } else {
-    L.xin = T(0);
-    L.xc = T(0);
+    L.xin = 0.f;
+    L.xc = 0.f;
   }
 }
 
 // Register windows along k.  Logical plane o (0 = newest) of step u lives in
 // physical slot (o + W - u % W) % W, so advancing one plane renames slots
 // instead of moving registers (the march is unrolled by W).
-template <typename T, int NU, int MODE>
+template <int NU, int MODE>
 struct CellState {
   static constexpr int H = 2 * NU, W = H + 2;
-  T xw[W], bw[W], dw[W], rdw[W], czw[W], cxw[W], cxmw[W], cyw[W], cymw[W];
+  float xw[W], bw[W], dw[W], rdw[W], czw[W], cxw[W], cxmw[W], cyw[W], cymw[W];
   bool dpos[W];  // d > 0 of each plane, tested once when the plane enters
-  T racc;
+  float racc;
   double dacc[2];  // CG dot products (finest post-smoother)
 };
 
 // One pipeline step: plane t enters (from L), half-sweeps on the planes
 // behind it, output/residual of plane t - H, restriction after the barrier.
 // U = position of this step in the W-step unrolled march (t - t0 = U mod W).
-template <typename T, int NU, int MODE, bool HAS_E, bool DOTS, int U, int EX, int EY>
-__device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L,
-                                  const FusedArgs<T>& A, const CellCol& C,
-                                  T (*xs)[EY + 2][EX + 2], T (*rs)[EY][EX], int t, int k0, int k1) {
+template <int NU, int MODE, bool HAS_E, bool DOTS, int U, int EX, int EY>
+__device__ inline void cell_step(CellState<NU, MODE>& F, const CellLoad& L,
+                                  const FusedArgs<float>& A, const CellCol& C,
+                                  float (*xs)[EY + 2][EX + 2], float (*rs)[EY][EX], int t,
+                                  int k0, int k1) {
   using Sh = CellShape<NU, EX, EY>;
   constexpr int H = Sh::H, W = Sh::W, R = Sh::R;
   static_assert(R == W && (W % 2) == 0, "ring slots are compile-time only for R == W, W even");
@@ -124,10 +113,10 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
   const bool outq = q >= k0 && q < k1;
   const bool wr = outq && C.tile && C.in_ij;
 
-  const T lb = L.vt ? L.b : T(0), lcx = L.vt ? L.cx : T(0), lcy = L.vt ? L.cy : T(0);
-  const T lcz = L.vt ? L.cz : T(0), le = L.vt ? L.e : T(0);
-  const T lcxm = (L.vt && C.vxm) ? L.cxm : T(0), lcym = (L.vt && C.vym) ? L.cym : T(0);
-  T d0 = lcxm;
+  const float lb = L.vt ? L.b : 0.f, lcx = L.vt ? L.cx : 0.f, lcy = L.vt ? L.cy : 0.f;
+  const float lcz = L.vt ? L.cz : 0.f, le = L.vt ? L.e : 0.f;
+  const float lcxm = (L.vt && C.vxm) ? L.cxm : 0.f, lcym = (L.vt && C.vym) ? L.cym : 0.f;
+  float d0 = lcxm;
   d0 = d0 + lcym;
   d0 = d0 + F.czw[S(1)];
   d0 = d0 + lcx;
@@ -136,12 +125,12 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
   // the diagonal-only term; without one the sum stays as it is (adding +0
   // to a sum of non-negative couplings changes nothing)
   if (HAS_E) d0 = d0 + le;
-  T x0 = T(0);
-  if (MODE == 1) x0 = d0 > T(0) ? L.xin + L.xc : T(0);
+  float x0 = 0.f;
+  if (MODE == 1) x0 = d0 > 0.f ? L.xin + L.xc : 0.f;
   F.bw[S(0)] = lb; F.cxw[S(0)] = lcx; F.cxmw[S(0)] = lcxm; F.cyw[S(0)] = lcy;
   F.cymw[S(0)] = lcym; F.czw[S(0)] = lcz; F.dw[S(0)] = d0; F.xw[S(0)] = x0;
-  F.dpos[S(0)] = d0 > T(0);
-  F.rdw[S(0)] = d0 > T(0) ? smoother_rcp(d0) : T(0);
+  F.dpos[S(0)] = d0 > 0.f;
+  F.rdw[S(0)] = d0 > 0.f ? smoother_rcp(d0) : 0.f;
   xs[Q(0)][ly][lx] = x0;
 
   // cells of this thread's colour move this step (t0 even, W even)
@@ -150,13 +139,13 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
   for (int s = 1; s <= H; ++s) {
     const int o = MODE == 0 ? s - 1 : s;
     // planes outside [0, nz) have d = 0 and stay 0, so no range test
-    T v;
+    float v;
     if (MODE == 0 && s == 1) {
       v = F.bw[S(0)] * F.rdw[S(0)];
     } else {
-      const T xW = xs[Q(o)][ly][lx - 1], xS = xs[Q(o)][ly - 1][lx];
-      const T xE = xs[Q(o)][ly][lx + 1], xN = xs[Q(o)][ly + 1][lx];
-      T acc = T(0);
+      const float xW = xs[Q(o)][ly][lx - 1], xS = xs[Q(o)][ly - 1][lx];
+      const float xE = xs[Q(o)][ly][lx + 1], xN = xs[Q(o)][ly + 1][lx];
+      float acc = 0.f;
       acc += F.cxmw[S(o)] * xW;
       acc += F.cymw[S(o)] * xS;
       acc += F.czw[S(o + 1)] * F.xw[S(o + 1)];
@@ -169,17 +158,17 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
     // keep v in a register on every lane: a select whose operand is only
     // needed on some lanes would otherwise become an exec-masked branch
     __asm__ volatile("" : "+v"(v));
-    const T xn = (act && F.dpos[S(o)]) ? v : F.xw[S(o)];
+    const float xn = (act && F.dpos[S(o)]) ? v : F.xw[S(o)];
     F.xw[S(o)] = xn;
     xs[Q(o)][ly][lx] = xn;
   }
 
   if (MODE == 0) {
-    T r = T(0);
+    float r = 0.f;
     if (wr && F.dpos[S(H)]) {
-      const T xW = xs[Q(H)][ly][lx - 1], xS = xs[Q(H)][ly - 1][lx];
-      const T xE = xs[Q(H)][ly][lx + 1], xN = xs[Q(H)][ly + 1][lx];
-      T acc = T(0);
+      const float xW = xs[Q(H)][ly][lx - 1], xS = xs[Q(H)][ly - 1][lx];
+      const float xE = xs[Q(H)][ly][lx + 1], xN = xs[Q(H)][ly + 1][lx];
+      float acc = 0.f;
       acc += F.cxmw[S(H)] * xW;
       acc += F.cymw[S(H)] * xS;
       acc += F.czw[S(H + 1)] * F.xw[S(H + 1)];
@@ -188,11 +177,11 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
       acc += F.czw[S(H)] * F.xw[S(H - 1)];
       r = F.bw[S(H)] - (F.dw[S(H)] * F.xw[S(H)] - acc);
     }
-    if (wr) cell_put(A.xout, C.col + C.plane * (uint32_t)q, F.xw[S(H)]);
+    if (wr) put_off(A.xout, C.col + C.plane * (uint32_t)q, F.xw[S(H)]);
     // q = t0 + U - H (mod W) with t0 and H even: parity of q = parity of U
     if (q >= 0) rs[U & 1][ty][tx] = r;
   } else if (wr) {
-    cell_put(A.xout, C.col + C.plane * (uint32_t)q, F.xw[S(H)]);
+    put_off(A.xout, C.col + C.plane * (uint32_t)q, F.xw[S(H)]);
     if (DOTS && A.dots) {
       const double z = (double)F.xw[S(H)];
       // (r, z) with the FP32 r the leg smooths with (the b window): an
@@ -205,7 +194,7 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
   lds_barrier();
   if (MODE == 0 && wr && ((tx - H) & 1) == 0 && ((ty - H) & 1) == 0) {
     constexpr int sl = U & 1;
-    T ps = rs[sl][ty][tx];
+    float ps = rs[sl][ty][tx];
     ps += rs[sl][ty][tx + 1];
     ps += rs[sl][ty + 1][tx];
     ps += rs[sl][ty + 1][tx + 1];
@@ -213,7 +202,7 @@ __device__ inline void cell_step(CellState<T, NU, MODE>& F, const CellLoad<T>& L
     F.racc = first ? ps : F.racc + ps;
     if (!first || q == A.nz - 1) {
       // C.ccol: byte offset of the coarse column (i/2, j/2)
-      cell_put(A.bc, C.ccol + C.cplane * (uint32_t)(q >> 1), F.racc);
+      put_off(A.bc, C.ccol + C.cplane * (uint32_t)(q >> 1), F.racc);
     }
   }
 }
@@ -232,29 +221,29 @@ constexpr int cell_pipe() {
 // path per step would merge into the loop head with fewer loads in flight,
 // and the compiler's wait counts there would drain the load pipeline on
 // every turn.
-template <typename T, int NU, int MODE, bool HAS_E, bool DOTS, bool CHECK, int U, int EX, int EY>
-__device__ inline void cell_march(CellState<T, NU, MODE>& F, CellLoad<T> (&LB)[cell_pipe<NU>()],
-                                   const FusedArgs<T>& A, const CellCol& C,
-                                   T (*xs)[EY + 2][EX + 2], T (*rs)[EY][EX], int t, int t1,
+template <int NU, int MODE, bool HAS_E, bool DOTS, bool CHECK, int U, int EX, int EY>
+__device__ inline void cell_march(CellState<NU, MODE>& F, CellLoad (&LB)[cell_pipe<NU>()],
+                                   const FusedArgs<float>& A, const CellCol& C,
+                                   float (*xs)[EY + 2][EX + 2], float (*rs)[EY][EX], int t, int t1,
                                    int k0, int k1) {
   if constexpr (U < CellShape<NU>::W) {
     if (CHECK && t + U >= t1) return;
     constexpr int P = cell_pipe<NU>();
     static_assert(CellShape<NU>::W % P == 0, "load buffers must tile the window");
-    CellLoad<T>& L = LB[U % P];
-    cell_step<T, NU, MODE, HAS_E, DOTS, U, EX, EY>(F, L, A, C, xs, rs, t + U, k0, k1);
-    cell_load<T, MODE, HAS_E>(L, A, C, t + U + P);
-    cell_march<T, NU, MODE, HAS_E, DOTS, CHECK, U + 1, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
+    CellLoad& L = LB[U % P];
+    cell_step<NU, MODE, HAS_E, DOTS, U, EX, EY>(F, L, A, C, xs, rs, t + U, k0, k1);
+    cell_load<MODE, HAS_E>(L, A, C, t + U + P);
+    cell_march<NU, MODE, HAS_E, DOTS, CHECK, U + 1, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   }
 }
 
-template <typename T, int NU, int MODE, bool FINE, bool HAS_E, int EX = kFEX, int EY = kFEY>
-__global__ void __launch_bounds__(EX * EY) k_smooth_cell(FusedArgs<T> A, const Scalars* S) {
+template <int NU, int MODE, bool FINE, bool HAS_E, int EX = kFEX, int EY = kFEY>
+__global__ void __launch_bounds__(EX * EY) k_smooth_cell(FusedArgs<float> A, const Scalars* S) {
   if (S->done) return;
   using Sh = CellShape<NU, EX, EY>;
   constexpr int H = Sh::H, TX = Sh::TX, TY = Sh::TY, W = Sh::W, R = Sh::R;
-  __shared__ T xs[R][EY + 2][EX + 2];
-  __shared__ T rs[2][EY][EX];
+  __shared__ float xs[R][EY + 2][EX + 2];
+  __shared__ float rs[2][EY][EX];
   uint32_t bx, by, bz;
   xcd_block3(bx, by, bz);
   CellCol C;
@@ -267,31 +256,32 @@ __global__ void __launch_bounds__(EX * EY) k_smooth_cell(FusedArgs<T> A, const S
   C.vxm = C.i > 0;
   C.vym = C.j > 0;
   C.act_even = ((C.i + C.j) & 1) == 0;
-  C.col = C.in_ij ? (uint32_t)(C.i + A.nx * C.j) * (uint32_t)sizeof(T) : 0u;
-  C.plane = (uint32_t)A.nx * (uint32_t)A.ny * (uint32_t)sizeof(T);
-  C.dxm = (C.in_ij && C.vxm) ? (uint32_t)sizeof(T) : 0u;
-  C.dym = (C.in_ij && C.vym) ? (uint32_t)(A.nx * sizeof(T)) : 0u;
-  C.ccol = C.in_ij ? (uint32_t)((C.i >> 1) + A.cnx * (C.j >> 1)) * (uint32_t)sizeof(T) : 0u;
-  C.cplane = (uint32_t)A.cnx * (uint32_t)A.cny * (uint32_t)sizeof(T);
+  C.col = C.in_ij ? (uint32_t)(C.i + A.nx * C.j) * (uint32_t)sizeof(float) : 0u;
+  C.plane = (uint32_t)A.nx * (uint32_t)A.ny * (uint32_t)sizeof(float);
+  C.dxm = (C.in_ij && C.vxm) ? (uint32_t)sizeof(float) : 0u;
+  C.dym = (C.in_ij && C.vym) ? (uint32_t)(A.nx * sizeof(float)) : 0u;
+  C.ccol = C.in_ij ? (uint32_t)((C.i >> 1) + A.cnx * (C.j >> 1)) * (uint32_t)sizeof(float) : 0u;
+  C.cplane = (uint32_t)A.cnx * (uint32_t)A.cny * (uint32_t)sizeof(float);
   const int k0 = (int)bz * A.kchunk;
   const int k1 = min(k0 + A.kchunk, A.nz);
 
-  CellState<T, NU, MODE> F;
+  CellState<NU, MODE> F;
 #pragma unroll
   for (int o = 0; o < W; ++o) {
     F.xw[o] = F.bw[o] = F.dw[o] = F.rdw[o] = F.czw[o] = F.cxw[o] = F.cxmw[o] = F.cyw[o] =
-        F.cymw[o] = T(0);
+        F.cymw[o] = 0.f;
     F.dpos[o] = false;
   }
-  F.racc = T(0);
+  F.racc = 0.f;
   F.dacc[0] = F.dacc[1] = 0.0;
-  for (int q = C.ty * EX + C.tx; q < R * (EY + 2) * (EX + 2); q += EX * EY) (&xs[0][0][0])[q] = T(0);
-  for (int q = C.ty * EX + C.tx; q < 2 * EY * EX; q += EX * EY) (&rs[0][0][0])[q] = T(0);
+  for (int q = C.ty * EX + C.tx; q < R * (EY + 2) * (EX + 2); q += EX * EY) (&xs[0][0][0])[q] = 0.f;
+  for (int q = C.ty * EX + C.tx; q < 2 * EY * EX; q += EX * EY) (&rs[0][0][0])[q] = 0.f;
   // cz of the plane below the first loaded one (bottom face of that plane):
   // logical plane 1 of the first step, physical slot 1
   {
     const int pb = k0 - H - 1;
-    if (C.in_ij && pb >= 0 && pb < A.nz) F.czw[1] = cell_at(A.cz, C.col + C.plane * (uint32_t)pb);
+    if (C.in_ij && pb >= 0 && pb < A.nz)
+      F.czw[1] = at_off<float>(A.cz, C.col + C.plane * (uint32_t)pb);
   }
   __syncthreads();
 
@@ -299,14 +289,14 @@ __global__ void __launch_bounds__(EX * EY) k_smooth_cell(FusedArgs<T> A, const S
   const int t0 = k0 - H, t1 = k1 + H;  // steps [t0, t1); t0 even
   constexpr int P = cell_pipe<NU>();
   constexpr bool DOTS = FINE && MODE == 1;
-  CellLoad<T> LB[P];
+  CellLoad LB[P];
 #pragma unroll
-  for (int u = 0; u < P; ++u) cell_load<T, MODE, HAS_E>(LB[u], A, C, t0 + u);
+  for (int u = 0; u < P; ++u) cell_load<MODE, HAS_E>(LB[u], A, C, t0 + u);
   int t = t0;
   for (; t + W <= t1; t += W)
-    cell_march<T, NU, MODE, HAS_E, DOTS, false, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
+    cell_march<NU, MODE, HAS_E, DOTS, false, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   if (t < t1)
-    cell_march<T, NU, MODE, HAS_E, DOTS, true, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
+    cell_march<NU, MODE, HAS_E, DOTS, true, 0, EX, EY>(F, LB, A, C, xs, rs, t, t1, k0, k1);
   if constexpr (DOTS) {
     if (A.dots) block_partials<EX * EY, 2, 0u>(A.dsite, F.dacc);
   }

@@ -1,4 +1,4 @@
-// Multigrid-preconditioned flexible CG on the GPU.
+// Multigrid-preconditioned CG on the GPU.
 //
 // Replaces HYPRE PCG + BoomerAMG (ProjectionP.f90:95-116, 267-299).  The
 // outer CG, its dot products and the residual are FP64; the V-cycle runs in
@@ -682,7 +682,8 @@ __device__ inline void set_direction(Scalars* S, int slot, double m, double rz, 
   if (!is_finite(rz) || !is_finite(beta)) { S->nonfinite = 1; S->done = 1; }
 }
 
-// rz = (r, z), zq = (z, q);  beta = -alpha zq / rz_old (flexible CG).
+// rz = (r, z), zq = (z, q);  beta = -alpha zq / rz_old: flexible CG, for the
+// preconditioners without fused dot products (k_cg_dots2_fin).
 // Singular systems: z is shifted by its diagonal-weighted mean m so the
 // iterate keeps the pressure of the stiff (high-coefficient) phase near zero;
 // (r, z-m) and (z-m, q) follow from the raw sums.
@@ -1051,11 +1052,11 @@ void launch_march(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int 
 #undef SP_K
 }
 
-template <typename T, int NU, bool HAS_E, int EX, int EY>
-void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int mode) {
+template <int NU, bool HAS_E, int EX, int EY>
+void launch_cell(sp_ctx* c, const Level<float>& L, FusedArgs<float>& A, bool fine, int mode) {
   const dim3 grd(L.leg.gx, L.leg.gy, L.leg.gz), blk(EX, EY, 1);
   const Scalars* S = c->S;
-#define SP_K(MODE, FINE) k_smooth_cell<T, NU, MODE, FINE, HAS_E, EX, EY>
+#define SP_K(MODE, FINE) k_smooth_cell<NU, MODE, FINE, HAS_E, EX, EY>
   SP_LEG(SP_K);
 #undef SP_K
 }
@@ -1064,13 +1065,13 @@ void launch_cell(sp_ctx* c, const Level<T>& L, FusedArgs<T>& A, bool fine, int m
 template <int NU>
 void launch_leg(sp_ctx* c, const Level<float>& L, FusedArgs<float>& A, bool fine, int mode) {
   if (small_legs(L, fine)) {
-    if (A.e) launch_cell<float, NU, true, kFEXs, kFEYs>(c, L, A, fine, mode);
-    else launch_cell<float, NU, false, kFEXs, kFEYs>(c, L, A, fine, mode);
+    if (A.e) launch_cell<NU, true, kFEXs, kFEYs>(c, L, A, fine, mode);
+    else launch_cell<NU, false, kFEXs, kFEYs>(c, L, A, fine, mode);
   } else if (L.four) {
     launch_march<float, NU, false, false>(c, L, A, fine, mode);
   } else {
-    if (A.e) launch_cell<float, NU, true, kFEX, kFEY>(c, L, A, fine, mode);
-    else launch_cell<float, NU, false, kFEX, kFEY>(c, L, A, fine, mode);
+    if (A.e) launch_cell<NU, true, kFEX, kFEY>(c, L, A, fine, mode);
+    else launch_cell<NU, false, kFEX, kFEY>(c, L, A, fine, mode);
   }
 }
 template <int NU>
@@ -1256,9 +1257,10 @@ sp_status setup_levels(sp_ctx* c, Level<T>* lv) {
 
 // The first level of the tail kernel (c->tail_level): the levels from it on
 // fit its threads (two pairs each on the first level, one on the others; four
-// on a coarsest level alone in FP32) and LDS.  c->levels when not even the coarsest level does (a hierarchy cut short
-// by mg_levels, or a large grid that cannot coarsen): the V-cycle then smooths
-// the coarsest level in global memory.
+// on a coarsest level alone in FP32) and LDS.  c->levels when not even the
+// coarsest level does (a hierarchy cut short by mg_levels, or a large grid
+// that cannot coarsen): the V-cycle then smooths the coarsest level in global
+// memory.
 template <typename T>
 static int first_tail_level(const Level<T>* lv, int levels) {
   int best = levels;
@@ -1287,8 +1289,8 @@ sp_status mg_setup(sp_ctx* c) {
   return setup_levels<double>(c, c->ld);
 }
 
-// Solve A x = rhs - mean (singular) with the multigrid-preconditioned
-// flexible CG until max |r_i| / V_i <= tol.  The operator arrays and c->S
+// Solve A x = rhs - mean (singular) with the preconditioned
+// CG until max |r_i| / V_i <= tol.  The operator arrays and c->S
 // (bmean, singular) come from the assembly.  Writes x into c->x.
 //   check_true: after convergence of the recursive residual, form the true
 //               residual and restart from it (at most 3 times) if it is
