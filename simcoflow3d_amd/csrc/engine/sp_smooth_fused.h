@@ -62,8 +62,10 @@ struct FusedArgs {
 
 // The extended tile of a leg (threads along i x rows) and pairs per thread.
 //
-// The leg is bound by the lines it pulls through L2 (its extended tiles, 1.7 to
-// 1.9 times the interior) and by the step's instruction stream, about evenly.
+// No unit is saturated at 256^3 (counters): 1.2 to 1.3 times the algorithmic
+// bytes at 0.75 to 0.9 of the copy rate, the VALU a third busy; waits for loads
+// and the barrier (about 40 % of a wave's cycles) and for issue (30 %) overlap
+// only in part, for want of waves.
 // FP32: four cells per thread with 16-byte loads (256 VGPRs, two waves per
 // SIMD), a 64 x 16 interior whose rows are whole cache lines; measured at
 // 256^3 with one cell per thread and a 32 x 16 interior 117 (pre) and 140 us
