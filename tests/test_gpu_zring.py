@@ -75,3 +75,25 @@ def test_bytes_of_the_pass_that_forms_x(gpu_available, prec, depth):
     full = t["launches"] - 1  # passes that keep p: it is written, and read by the next
     assert full == st.iterations // depth  # one more step was under way
     assert t["bytes"] == n * (z * st.iterations + 9 + full * (9 + 8 + 8 + 8))
+
+
+@pytest.mark.parametrize("prec", (0, 1))
+def test_adjoint_after_the_ring_was_given_back(gpu_available, prec):
+    """The ring may go between a forward and its adjoint: the same gradients."""
+    c = H.case(2, size=(33, 20, 26))
+    print(f"[zring] adjoint prec={prec}", flush=True)
+    g = []
+    for q in range(3):
+        a = np.zeros(c.halo_shape, order="F")
+        a[1:-1, 1:-1, 1:-1] = np.random.default_rng(q).uniform(0.0, 1.0, c.shape)
+        g.append(a)
+    P = H.projector(c, precision=prec, mg_levels=2)
+    P.project(H.fields(c), c.bc_flag, c.dt)
+    first, st = P.adjoint(*g)
+    P.set_solver_memory(0)
+    second, st2 = P.adjoint(*g)
+    P.close()
+    assert st.iterations == st2.iterations > 16
+    for n in first:
+        if first[n] is not None:
+            assert np.array_equal(first[n], second[n]), n
